@@ -20,136 +20,10 @@ struct CodecArgs {
     const float* rope_dm;
     const float* rope_dp;
     uint32_t heads, seq, n_tensors, bh, work, per_xcd;
+    // dequant_kernel: 64-token tiles, (tensor, batch x head) streams, streams per block, nontemporal stores
+    uint32_t n_tiles, n_sub, group, stream_out;
     float hscale;
 };
-
-// Lattice points of this lane's C groups from the packed row.
-template <int D, int L>
-__device__ __forceinline__ void unpack_points(const CodecArgs& a, uint32_t tensor, size_t row, int q,
-                                             float (&p)[D / 32][8], int (&coset)[D / 32], float& scale) {
-    constexpr int C = D / 32;
-    constexpr int B = SymBits<L>::value;
-    constexpr int NB = C * B;
-    constexpr int HL = L / 2;
-    constexpr int ROW_BYTES = D / 8 * B;
-    const uint8_t* src = reinterpret_cast<const uint8_t*>(a.syms[tensor]) + row * ROW_BYTES + q * NB;
-    uint8_t bytes[NB];
-    if constexpr (NB % 4 == 0) {
-#pragma unroll
-        for (int k = 0; k < NB; k += 4) {
-            uint32_t w = *reinterpret_cast<const uint32_t*>(src + k);
-            bytes[k] = (uint8_t)w;
-            bytes[k + 1] = (uint8_t)(w >> 8);
-            bytes[k + 2] = (uint8_t)(w >> 16);
-            bytes[k + 3] = (uint8_t)(w >> 24);
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < NB; k += 2) {
-            uint16_t w = *reinterpret_cast<const uint16_t*>(src + k);
-            bytes[k] = (uint8_t)w;
-            bytes[k + 1] = (uint8_t)(w >> 8);
-        }
-    }
-    const uint8_t* cb = reinterpret_cast<const uint8_t*>(a.cosets[tensor]) + row * (D / 64);
-    uint32_t cbits;
-    if constexpr (D == 64) cbits = *cb;
-    else if constexpr (D == 128) cbits = *reinterpret_cast<const uint16_t*>(cb);
-    else cbits = *reinterpret_cast<const uint32_t*>(cb);
-    scale = reinterpret_cast<const float*>(a.scales[tensor])[row];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        uint64_t v = 0;
-#pragma unroll
-        for (int m = 0; m < B; ++m) v |= (uint64_t)bytes[c * B + m] << (8 * m);
-        coset[c] = (int)((cbits >> (4 * c + q)) & 1u);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int sym = (int)((v >> (B * j)) & ((1u << B) - 1u));
-            float x = (float)(sym - HL);
-            if (coset[c]) {
-                if constexpr ((HL & 1) == 0) x = __builtin_fminf(x + 0.5f, (float)HL);
-                else x = __builtin_fmaxf(x - 0.5f, (float)-HL);
-            }
-            p[c][j] = x;
-        }
-    }
-}
-
-template <int D, int L, bool IS_KEY, int DR>
-__global__ __launch_bounds__(256) void dequant_kernel(CodecArgs a) {
-    constexpr int C = D / 32;
-    constexpr int RC = RopeChunks<D, DR>::value;
-    const int q = threadIdx.x & 3;
-    const uint32_t w = (blockIdx.x & 7u) * a.per_xcd + (blockIdx.x >> 3);
-    if (w >= a.work) return;
-    const uint32_t tensor = w % a.n_tensors;
-    const uint32_t rest = w / a.n_tensors;
-    const uint32_t bh = rest % a.bh;
-    const uint32_t t_raw = (rest / a.bh) * 64u + (threadIdx.x >> 2);
-    const bool active = t_raw < a.seq;
-    const uint32_t t = active ? t_raw : a.seq - 1u;
-    const size_t row = (size_t)bh * a.seq + t;
-
-    float x[C][8];
-    int coset[C];
-    float scale;
-    unpack_points<D, L>(a, tensor, row, q, x, coset, scale);
-    const float g = quad_sign(q) * (a.hscale * scale);
-    // keys with DR == D: the top Hadamard stage merges with forward RoPE, as in
-    // the quantizer (the sum of exact partial transforms is the same number)
-    constexpr bool MERGED = IS_KEY && DR == D;
-    constexpr bool EXACT_F16 = D * (L / 2) <= 1024;
-    if constexpr (EXACT_F16) {
-        half2v hp[C][4];
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                hp[c][k] = __builtin_bit_cast(half2v, __builtin_amdgcn_cvt_pkrtz(x[c][2 * k], x[c][2 * k + 1]));
-        fwht_row_f16<C, !MERGED>(hp, q);
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                x[c][2 * k] = __builtin_fmaf((float)hp[c][k].x, g, 0.0f);
-                x[c][2 * k + 1] = __builtin_fmaf((float)hp[c][k].y, g, 0.0f);
-            }
-    } else {
-        fwht_row<C, !MERGED>(x, q);
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) x[c][i] = x[c][i] * g;
-    }
-    if constexpr (MERGED) {
-        float dm[RC][8], dp[RC][8];
-        load_rope_merged<D>(a.rope_cos, a.rope_sin, a.rope_dm, a.rope_dp, t, q, dm, dp);
-        rope_stage_merged<C>(x, dm, dp);
-    } else if constexpr (IS_KEY) {
-        float cs[RC][8], sn[RC][8];
-        load_rope<D, DR, RC>(a.rope_cos, a.rope_sin, t, q, cs, sn);
-        apply_rope<D, DR, RC, false>(x, q, cs, sn);
-    }
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) asm("" : "+v"(x[c][i]));  // keep the fp32 rounding (see quantizer)
-    if (!active) return;
-    half2v* dst = reinterpret_cast<half2v*>(reinterpret_cast<uint16_t*>(a.out[tensor]) + row * DR);
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        if (32 * c >= DR) continue;
-        uint4 o;
-        half2v h0 = {(__fp16)x[c][0], (__fp16)x[c][1]}, h1 = {(__fp16)x[c][2], (__fp16)x[c][3]};
-        half2v h2 = {(__fp16)x[c][4], (__fp16)x[c][5]}, h3 = {(__fp16)x[c][6], (__fp16)x[c][7]};
-        o.x = __builtin_bit_cast(uint32_t, h0);
-        o.y = __builtin_bit_cast(uint32_t, h1);
-        o.z = __builtin_bit_cast(uint32_t, h2);
-        o.w = __builtin_bit_cast(uint32_t, h3);
-        *reinterpret_cast<uint4*>(dst + (32 * c + 8 * q) / 2) = o;
-    }
-}
 
 // ---------------------------------------------------------------------------
 // int8 2p codes straight from the packed symbols, in integer arithmetic.  A
@@ -227,9 +101,9 @@ struct RowSyms {
     uint32_t d[(NB + 3) / 4];
     uint32_t cbits;
 
-    __device__ __forceinline__ void load(const CodecArgs& a, uint32_t tensor, size_t row, int q) {
+    __device__ __forceinline__ void load(uint64_t syms, uint64_t cosets, size_t row, int q) {
         constexpr int ND = (NB + 3) / 4;
-        const uint8_t* src = reinterpret_cast<const uint8_t*>(a.syms[tensor]) + row * (D / 8 * SymBits<L>::value) + q * NB;
+        const uint8_t* src = gptr<const uint8_t>(syms) + row * (D / 8 * SymBits<L>::value) + q * NB;
         if constexpr (NB % 4 == 0) {
 #pragma unroll
             for (int k = 0; k < ND; ++k) d[k] = reinterpret_cast<const uint32_t*>(src)[k];
@@ -241,7 +115,7 @@ struct RowSyms {
                 d[k] = lo16 | (hi16 << 16);
             }
         }
-        const uint8_t* cb = reinterpret_cast<const uint8_t*>(a.cosets[tensor]) + row * (D / 64);
+        const uint8_t* cb = gptr<const uint8_t>(cosets) + row * (D / 64);
         if constexpr (D == 64) cbits = *cb;
         else if constexpr (D == 128) cbits = *reinterpret_cast<const uint16_t*>(cb);
         else cbits = *reinterpret_cast<const uint32_t*>(cb);
@@ -251,8 +125,182 @@ struct RowSyms {
 template <int D, int L>
 __device__ __forceinline__ void codes_to_row(const CodecArgs& a, uint32_t tensor, size_t row, int q, uint8_t* lds_row) {
     RowSyms<D, L> rs;
-    rs.load(a, tensor, row, q);
+    rs.load(a.syms[tensor], a.cosets[tensor], row, q);
     groups_to_row<D, L>(rs.d, rs.cbits, q, lds_row);
+}
+
+// The codes 2p of this lane's group c as fp16 pairs, register k holding
+// coordinates k and k + 4.  A symbol s placed at mantissa bit 4 of 0x5400 is the
+// fp16 number 64 + s, and 2 (64 + s) - 128 - L (+1 or -1 in the half coset) is 2p
+// before its cap (floor), every step exact for any symbol value.
+template <int D, int L, int c>
+__device__ __forceinline__ void group_2p(const uint32_t (&d)[(D / 32 * SymBits<L>::value + 3) / 4], uint32_t cbits, int q,
+                                         half2v (&h)[4]) {
+    constexpr int B = SymBits<L>::value;
+    constexpr bool UP = ((L / 2) & 1) == 0;
+    const bool half = ((cbits >> (4 * c + q)) & 1u) != 0;
+    const __fp16 bias = half ? (__fp16)(UP ? -127.0f - L : -129.0f - L) : (__fp16)(-128.0f - L);
+    const __fp16 cap = half ? (__fp16)(UP ? L : -L) : (__fp16)(UP ? 65504.0f : -65504.0f);
+    const half2v two = {(__fp16)2.0f, (__fp16)2.0f}, bias2 = {bias, bias}, cap2 = {cap, cap};
+    uint32_t y[4];
+    if constexpr (B == 5) {
+        const uint32_t lo = window32<8 * B * c>(d), hi = window32<8 * B * c + 4 * B>(d);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            y[k] = (((lo >> (B * k)) & 31u) << 4) | (((hi >> (B * k)) & 31u) << 20) | 0x54005400u;
+    } else {
+        uint32_t x;  // symbols k and k + 4 at bits B k and B k + 16
+        if constexpr (B == 4) x = d[c];
+        else x = (window32<8 * B * c>(d) & ((1u << (4 * B)) - 1u)) | (window32<8 * B * c + 4 * B>(d) << 16);
+        constexpr uint32_t M = ((1u << B) - 1u) * 0x00100010u;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) y[k] = ((B * k < 4 ? x << (4 - B * k) : x >> (B * k - 4)) & M) | 0x54005400u;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const half2v v = __builtin_elementwise_fma(__builtin_bit_cast(half2v, y[k]), two, bias2);
+        h[k] = UP ? __builtin_elementwise_min(v, cap2) : __builtin_elementwise_max(v, cap2);
+    }
+}
+
+template <int D, int L, int c = 0>
+__device__ __forceinline__ void row_2p(const uint32_t (&d)[(D / 32 * SymBits<L>::value + 3) / 4], uint32_t cbits, int q,
+                                       half2v (&h)[D / 32][4]) {
+    if constexpr (c < D / 32) {
+        group_2p<D, L, c>(d, cbits, q, h[c]);
+        row_2p<D, L, c + 1>(d, cbits, q, h);
+    }
+}
+
+// One stream per block: values, which share no RoPE rows, and keys of head_dim
+// 256, whose RoPE rows would take 64 registers a lane (8 layers x 8 heads x 16384
+// tokens: 279 us with the rows held, 199 with them loaded per row, 203 before).
+template <int D, bool IS_KEY>
+constexpr bool dequant_one_stream() { return !IS_KEY || D == 256; }
+
+// fp16 reconstructions of packed rows.  A block owns one 64-token tile (a quad
+// per token), keeps the tile's RoPE rows in registers and walks `group` of the
+// (tensor, batch x head) streams, the next stream's symbols, coset bits and
+// scale (6 registers at D = 128) in flight during the current one.  The codes
+// stay packed fp16 up to the scale: the integers 2p and their Walsh-Hadamard
+// sums (at most D L) are exact, so with half the scale the results equal the
+// quantizer's own reconstruction bit for bit.
+// Blocks take the tile fastest, so those resident on an XCD stream a few
+// contiguous regions; the tile's RoPE rows are read once per group.
+// What bounds it: the stores.  One stream per block through unpack, transform and
+// RoPE in fp32 with quad stores took 116 us (keys) and 89 us (values) for the 341
+// and 325 MB of 4 layers x 8 heads x 32768 tokens; this form takes 84 and 77
+// between events (4.1 and 4.2 TB/s), of which the whole-line stores of
+// store_rows16 are 105 -> 91 us (keys) and nontemporal stores 91 -> 84.  Keys of
+// head_dim 96 (4 x 32 heads x 16384) 209 -> 140, of 64 (4 x 8 x 32768) 66 -> 42.
+template <int D, int L, bool IS_KEY, int DR>
+__global__ __launch_bounds__(256) void dequant_kernel(CodecArgs a, const uint64_t* __restrict__ syms,
+                                                      const uint64_t* __restrict__ cosets,
+                                                      const uint64_t* __restrict__ scales,
+                                                      const uint64_t* __restrict__ outs) {
+    constexpr int C = D / 32;
+    constexpr int RC = RopeChunks<D, DR>::value;
+    // keys with DR == D: the top Hadamard stage merges with forward RoPE, as in
+    // the quantizer (the sum of exact partial transforms is the same number)
+    constexpr bool MERGED = IS_KEY && DR == D;
+    constexpr bool EXACT_F16 = D * (L / 2) <= 1024;
+    constexpr bool ONE = dequant_one_stream<D, IS_KEY>();
+    const int q = threadIdx.x & 3;
+    const uint32_t w = (blockIdx.x & 7u) * a.per_xcd + (blockIdx.x >> 3);
+    if (w >= a.work) return;
+    const uint32_t t_raw = (ONE && IS_KEY ? w / a.n_sub : w % a.n_tiles) * 64u + (threadIdx.x >> 2);
+    const uint32_t t = min(t_raw, a.seq - 1u);
+    const uint32_t t0w = t_raw - ((threadIdx.x & 63u) >> 2);  // the wave's first token
+    if (t0w >= a.seq) return;                                  // no barrier follows
+    __shared__ uint4 stage[4][16 * (DR / 8)];
+    const uint32_t j0 = ONE ? (IS_KEY ? w % a.n_sub : w / a.n_tiles) : (w / a.n_tiles) * a.group;
+    const uint32_t j1 = ONE ? j0 + 1 : min(j0 + a.group, a.n_sub);
+    uint32_t tensor = j0 / a.bh, bh = j0 % a.bh;
+
+    float rope0[IS_KEY ? RC : 1][8], rope1[IS_KEY ? RC : 1][8];  // dm, dp or cos, sin
+    RowSyms<D, L> cur;
+    cur.load(syms[tensor], cosets[tensor], (size_t)bh * a.seq + t, q);
+    float scale = gptr<const float>(scales[tensor])[(size_t)bh * a.seq + t];
+    auto load_tables = [&]() {
+        if constexpr (MERGED) load_rope_merged<D>(a.rope_cos, a.rope_sin, a.rope_dm, a.rope_dp, t, q, rope0, rope1);
+        else if constexpr (IS_KEY) load_rope<D, DR, RC>(a.rope_cos, a.rope_sin, t, q, rope0, rope1);
+    };
+    if constexpr (!ONE) load_tables();
+
+    // the first row and the RoPE rows are waited for here: a wait inside the loop
+    // for loads of its entry would on every pass wait for the stores too
+    if constexpr (!ONE) {
+        for (uint32_t& v : cur.d) asm volatile("" : "+v"(v));
+        asm volatile("" : "+v"(cur.cbits), "+v"(scale));
+        if constexpr (IS_KEY) {
+#pragma unroll
+            for (int c = 0; c < RC; ++c)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(rope0[c][i]), "+v"(rope1[c][i]));
+        }
+    }
+    for (uint32_t j = j0; j < j1; ++j) {
+        const uint32_t tensor_c = tensor, bh_c = bh;
+        const uint32_t last = j + 1 < j1 ? 0u : 1u;  // the last pass loads its own row again (in bounds, unused)
+        if (!last && ++bh == a.bh) {
+            bh = 0;
+            ++tensor;
+        }
+        RowSyms<D, L> next;
+        float next_scale = 0.0f;
+        if constexpr (!ONE) {
+            next.load(syms[tensor], cosets[tensor], (size_t)bh * a.seq + t, q);
+            next_scale = gptr<const float>(scales[tensor])[(size_t)bh * a.seq + t];
+        }
+
+        half2v hp[C][4];
+        row_2p<D, L>(cur.d, cur.cbits, q, hp);
+        const float g = quad_sign(q) * (0.5f * (a.hscale * scale));
+        float x[C][8];
+        if constexpr (EXACT_F16) {
+            // the pairs are (k, k + 4) where fwht_row_f16 names them (2k, 2k + 1): its
+            // three in-chunk stages cover the same three index bits, in another order
+            fwht_row_f16<C, !MERGED>(hp, q);
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    x[c][k] = __builtin_fmaf((float)hp[c][k].x, g, 0.0f);
+                    x[c][k + 4] = __builtin_fmaf((float)hp[c][k].y, g, 0.0f);
+                }
+        } else {
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    x[c][k] = (float)hp[c][k].x;
+                    x[c][k + 4] = (float)hp[c][k].y;
+                }
+            fwht_row<C, !MERGED>(x, q);
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[c][i] = x[c][i] * g;
+        }
+        if constexpr (ONE) load_tables();
+        if constexpr (MERGED) rope_stage_merged<C>(x, rope0, rope1);
+        else if constexpr (IS_KEY) apply_rope<D, DR, RC, false>(x, q, rope0, rope1);
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) asm("" : "+v"(x[c][i]));  // keep the fp32 rounding (see quantizer)
+        uint32_t o[C][4];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) o[c][k] = __builtin_bit_cast(uint32_t, half2v{(__fp16)x[c][2 * k], (__fp16)x[c][2 * k + 1]});
+        store_rows16<DR>(gptr<uint8_t>(outs[tensor_c]) + ((size_t)bh_c * a.seq + t0w) * (2 * DR), min(16u, a.seq - t0w), o,
+                         stage[threadIdx.x >> 6], a.stream_out != 0);
+        if constexpr (!ONE) {
+            cur = next;
+            scale = next_scale;
+        }
+    }
 }
 
 // Byte-wise wrapping subtraction of four int8 lanes.
@@ -301,11 +349,11 @@ __global__ __launch_bounds__(256) void int8_codes_kernel(CodecArgs a) {
     // this thread's row of the next tile is loaded while the current one is
     // decoded and stored (rows past the stream read its last row, unused)
     RowSyms<D, L> next;
-    next.load(a, tensor, row0 + min(t_begin + r, a.seq - 1u), q);
+    next.load(a.syms[tensor], a.cosets[tensor], row0 + min(t_begin + r, a.seq - 1u), q);
     for (uint32_t t0 = t_begin; t0 < t_end; t0 += 64) {
         const uint32_t n_rows = min(64u, t_end - t0);
         const RowSyms<D, L> cur = next;
-        if (t0 + 64 < t_end) next.load(a, tensor, row0 + min(t0 + 64 + r, a.seq - 1u), q);
+        if (t0 + 64 < t_end) next.load(a.syms[tensor], a.cosets[tensor], row0 + min(t0 + 64 + r, a.seq - 1u), q);
         if (r < n_rows) groups_to_row<D, L>(cur.d, cur.cbits, q, tile + (r + 1) * STRIDE);
         __syncthreads();
         uint4 last = make_uint4(0u, 0u, 0u, 0u);
@@ -542,10 +590,23 @@ static hipError_t launch_delta_decode(const uint64_t* deltas, const uint64_t* ou
 
 template <int D, int L, int DR>
 static hipError_t launch_codec(int kind, bool key, const CodecArgs& a, hipStream_t s) {
-    dim3 grid(a.per_xcd * 8u);
     if (kind == 0) {
-        if (key) hipLaunchKernelGGL((dequant_kernel<D, L, true, DR>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((dequant_kernel<D, L, false, DR>), grid, dim3(256), 0, s, a);
+        CodecArgs b = a;
+        b.n_tiles = (a.seq + 63u) / 64u;
+        b.n_sub = a.bh * a.n_tensors;
+        // Keys: up to 16 streams share a block's RoPE rows (4 layers x 8 heads x
+        // 32768 tokens, K3: 131 us at 1 stream, 95 at 4, 87 at 8, 84 at 16, 88 at
+        // 32), fewer while the launch would have less than 1024 blocks.  Values
+        // have nothing to share: one stream each (77 us; 82 at 4 and 8).
+        const uint64_t all = (uint64_t)b.n_sub * b.n_tiles;
+        const bool one = key ? dequant_one_stream<D, true>() : dequant_one_stream<D, false>();
+        b.group = one ? 1u : (uint32_t)std::min<uint64_t>(std::max<uint64_t>(all / 1024, 1), 16);
+        b.stream_out = (uint64_t)a.n_tensors * a.bh * a.seq * DR * 2 >= kStreamBytes;
+        b.work = (b.n_sub + b.group - 1) / b.group * b.n_tiles;
+        b.per_xcd = (b.work + 7u) / 8u;
+        dim3 grid(b.per_xcd * 8u);
+        if (key) hipLaunchKernelGGL((dequant_kernel<D, L, true, DR>), grid, dim3(256), 0, s, b, b.syms, b.cosets, b.scales, b.out);
+        else hipLaunchKernelGGL((dequant_kernel<D, L, false, DR>), grid, dim3(256), 0, s, b, b.syms, b.cosets, b.scales, b.out);
     } else {
         // int8 codes: blocks of kInt8Tiles tiles of one stream
         CodecArgs b = a;

@@ -142,3 +142,26 @@ def test_c2_shaped_layer_properties_over_every_row():
         assert torch.equal(rans_decode(st), c)
         del x, rec, cd, back, c, d, st
         torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("D,L,key,n_t,shape", [
+    (128, 8, True, 5, (1, 7, 1000)),     # groups of several streams, the last one shorter; a cut tile
+    (128, 8, True, 3, (2, 4, 17)),       # one tile whose last waves hold one row and none
+    (128, 4, False, 2, (1, 3, 129)),
+    (96, 8, True, 2, (1, 5, 70)),
+    (64, 2, True, 3, (1, 2, 1)),
+    (64, 16, False, 2, (1, 2, 63)),
+    (256, 2, True, 2, (1, 3, 65)),
+    (128, 8, True, 33, (1, 8, 640)),     # enough streams and bytes for full groups and nontemporal stores
+])
+def test_dequantize_many_streams(D, L, key, n_t, shape):
+    """Several tensors per launch, streams grouped per block, rows that do not fill a wave's 16."""
+    from nexusquant_amd.codec import dequantize
+    from nexusquant_amd.ops import quantize_tensors
+    print(f"[gpu] dequant streams D={D} L={L} key={key} n={n_t} {shape}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(D + L + n_t)
+    xs = [torch.randn(*shape, D, generator=g, device=DEV).half() for _ in range(n_t)]
+    rec, cd = quantize_tensors(xs, is_key=key, levels=L, rope_base=10000.0, codes=True)
+    out = dequantize(cd, rope_base=10000.0)
+    torch.cuda.synchronize()
+    assert all(_same_fp16(o, r) for o, r in zip(out, rec))
