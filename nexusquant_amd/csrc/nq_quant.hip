@@ -61,6 +61,7 @@ extern "C" int nq_quantize(const nq_quant_desc* d, void* stream) {
     a.keep_mode = d->keep_mode;
     a.n_tensors = (uint32_t)d->n_tensors;
     a.batch = (uint32_t)d->batch;
+    a.stream_out = rows * a.n_tensors * (uint64_t)d->head_dim * 2 >= kStreamBytes;
     const uint64_t work = plan_work(a, (uint64_t)(d->seq_out + 63) / 64, d->is_key ? kKeyGroup : kMaxGroup,
                                     d->is_key && d->gather ? kGatherKeyMinBlocks : kMinBlocks);
     NQ_CHECK_ARG(work + 8 <= max_blocks(256), "nq_quantize: %llu work items exceed the grid limit",

@@ -59,6 +59,7 @@ struct QuantArgs {
     // the n_kept[b] kept ones first; output row = source row = the listed position
     const int32_t* order;
     const int32_t* n_kept;
+    uint32_t stream_out;                    // the reconstructions are stored nontemporally
 };
 
 // ------------------------------------------------------------------ E8 ----
@@ -339,12 +340,66 @@ struct RowOut {
     uint16_t* scales16;
 };
 
+// Whole-line stores of a wave's 16 reconstructed rows.  In the quad layout a
+// store instruction writes 16 runs of 64 bytes, half a cache line each; through
+// the wave's LDS buffer (swizzled as in store_rows16) it writes whole rows, 16
+// bytes a lane: instruction i stores 16-byte unit k of the wave's row rr, with
+// (rr, k) = divmod(64 i + lane, 16-byte units of a row).  row[i] is that row's token in
+// the output and act bit i whether this launch writes it.
+// Measured (bit-identical outputs; a call's time): 16 layers x K, V fp16 [4, 8, 8192,
+// 128] evicted at 25 %: 847 -> 811 us; 4 layers bf16 [1, 8, 131072, 128] with codes
+// 1006 -> 979; 4 layers of 65521 tokens truncated at 25 %: 759 -> 726.  The rest is
+// VALU issue: about 1080 instructions per 16 rows.
+template <int DR>
+struct WideRows {
+    static constexpr int UR = DR / 8;   // 16-byte units per row
+    static constexpr int N = DR / 32;   // store instructions (and chunks)
+    uint4* lds;
+    uint32_t row[N];
+    uint32_t act;
+    bool all;  // every unit of the wave's rows is written
+
+    static __device__ __forceinline__ int slot(int r, int k) { return r * UR + (UR % 16 == 0 ? k ^ (4 * (r & 3)) : k); }
+
+    __device__ __forceinline__ void init(uint4* wave_lds, uint32_t t_out, bool active) {
+        const int lane = threadIdx.x & 63;
+        lds = wave_lds;
+        act = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int src = 4 * ((64 * i + lane) / UR);  // the quad that owns the row
+            row[i] = (uint32_t)__shfl((int)t_out, src, 64);
+            act |= (uint32_t)__shfl(active ? 1 : 0, src, 64) << i;
+        }
+        all = __ballot(active) == ~0ull;
+    }
+
+    __device__ __forceinline__ void store(uint16_t* recon, uint32_t row0, const u32x4 (&v)[N], bool stream) const {
+        const int lane = threadIdx.x & 63;
+        u32x4* d[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            d[i] = reinterpret_cast<u32x4*>(recon) + (size_t)(row0 + row[i]) * UR + (64 * i + lane) % UR;
+        if (all && stream) {
+            asm volatile("" ::: "memory");  // keeps the branches' stores apart: merged, they lose the hint
+#pragma unroll
+            for (int i = 0; i < N; ++i) __builtin_nontemporal_store(v[i], d[i]);
+            asm volatile("" ::: "memory");
+        } else {
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if ((act >> i) & 1u) *d[i] = v[i];
+        }
+    }
+};
+
 // The row computation of one sub-item: x holds the source row (zero padded,
 // zeroed for evicted rows); cs / sn the source position's RoPE rows for keys.
 // With a gather list the forward rotation takes the output position's rows:
 // co / so for the merged layout, loaded per sub-item for the padded one.
-template <int D, int L, bool IS_KEY, int DR, bool PAGE, bool GATHER>
-__device__ __forceinline__ void quant_row_body(const QuantArgs& a, float (&x)[D / 32][8],
+// WIDE: the reconstruction leaves through `wide`.
+template <int D, int L, bool IS_KEY, int DR, bool PAGE, bool GATHER, bool WIDE>
+__device__ __forceinline__ void quant_row_body(const QuantArgs& a, const WideRows<DR>& wide, float (&x)[D / 32][8],
                                                float (&cs)[RopeChunks<D, DR>::value][8],
                                                float (&sn)[RopeChunks<D, DR>::value][8],
                                                const float (&co)[RopeChunks<D, DR>::value][8],
@@ -548,8 +603,6 @@ __device__ __forceinline__ void quant_row_body(const QuantArgs& a, float (&x)[D 
             apply_rope<D, DR, RC, false>(x, q, cs, sn);
         }
     }
-    if (!active) return;
-    uint16_t* dst = o.recon + out_row * DR;
     // The fp32 result is rounded to fp16 in a second step, as the reference does
     // (fp32 tensor, then .half()).  The empty asm pins the fp32 value: without it
     // the backend folds fma + convert into v_fma_mix{lo,hi}_f16, which rounds
@@ -558,18 +611,37 @@ __device__ __forceinline__ void quant_row_body(const QuantArgs& a, float (&x)[D 
     for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int i = 0; i < 8; ++i) asm("" : "+v"(x[c][i]));
+    uint4 w[DR / 32];
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
-        if (32 * c >= DR) continue;  // padding coordinates are not part of the output
+    for (int c = 0; c < DR / 32; ++c) {  // padding coordinates are not part of the output
         half2v hv[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) hv[k] = half2v{(__fp16)x[c][2 * k], (__fp16)x[c][2 * k + 1]};
-        uint4 w;
-        w.x = __builtin_bit_cast(uint32_t, hv[0]);
-        w.y = __builtin_bit_cast(uint32_t, hv[1]);
-        w.z = __builtin_bit_cast(uint32_t, hv[2]);
-        w.w = __builtin_bit_cast(uint32_t, hv[3]);
-        *reinterpret_cast<uint4*>(dst + 32 * c + 8 * q) = w;
+        w[c].x = __builtin_bit_cast(uint32_t, hv[0]);
+        w[c].y = __builtin_bit_cast(uint32_t, hv[1]);
+        w[c].z = __builtin_bit_cast(uint32_t, hv[2]);
+        w[c].w = __builtin_bit_cast(uint32_t, hv[3]);
+    }
+    if constexpr (WIDE) {
+        // the wave's own buffer: its LDS accesses execute in order, the barriers
+        // only keep the compiler from reordering them
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int c = 0; c < DR / 32; ++c) wide.lds[wide.slot(lane >> 2, 4 * c + q)] = w[c];
+        __builtin_amdgcn_wave_barrier();
+        u32x4 v[DR / 32];
+#pragma unroll
+        for (int i = 0; i < DR / 32; ++i) {
+            const int u = 64 * i + lane;
+            v[i] = *reinterpret_cast<const u32x4*>(&wide.lds[wide.slot(u / wide.UR, u % wide.UR)]);
+        }
+        __builtin_amdgcn_wave_barrier();
+        wide.store(o.recon, bh * a.seq_out, v, a.stream_out != 0);
+    } else {
+        if (!active) return;
+        uint16_t* dst = o.recon + out_row * DR;
+#pragma unroll
+        for (int c = 0; c < DR / 32; ++c) *reinterpret_cast<uint4*>(dst + 32 * c + 8 * q) = w[c];
     }
     }  // !PAGE
 }
@@ -578,16 +650,18 @@ __device__ __forceinline__ void quant_row_body(const QuantArgs& a, float (&x)[D 
 // or transforming it: a zeroed row quantizes to the integer point 0 (every
 // symbol L/2, coset bits 0), its amax is clamped to 1e-8, so its scale is
 // 1e-8 * (2/L) (exact: 2/L is a power of two), and its reconstruction is 0.
-// Same lanes and store widths as quant_row_body's stores.
+// Every lane of a wave calls it: reconstructions leave as whole rows, the other
+// outputs on the lanes and in the widths of quant_row_body's stores.
 template <int D, int L, int DR>
-__device__ __forceinline__ void store_evicted_row(const RowOut& o, size_t out_row, int q) {
+__device__ __forceinline__ void store_evicted_row(const RowOut& o, const WideRows<DR>& wide, uint32_t row0, uint32_t t_out,
+                                                  int q, bool active, bool stream) {
     constexpr int C = D / 32;
     if (o.recon) {
-        uint16_t* dst = o.recon + out_row * DR;
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-            if (32 * c < DR) *reinterpret_cast<uint4*>(dst + 32 * c + 8 * q) = make_uint4(0u, 0u, 0u, 0u);
+        u32x4 zero[DR / 32] = {};
+        wide.store(o.recon, row0, zero, stream);
     }
+    if (!active) return;
+    const size_t out_row = row0 + t_out;
     if (o.syms) {
         float p[C][8];
         int cs[C];
@@ -681,6 +755,10 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
     uint32_t t_out = in_range ? t_raw : a.seq_out - 1u;  // idle quads recompute a valid row
     uint32_t t_in = t_out;
     bool keep = true;
+    // Whole-line stores of the reconstructions; keys with the padded RoPE layout
+    // keep the quad stores (their RoPE rows already take 24 KB of LDS a block).
+    constexpr bool WIDE = !PAGE && !(IS_KEY && DR != D);
+    WideRows<DR> wide;
     if constexpr (LIST) {
         // Row list: entry t_raw of the batch row's list; the first n_kept are kept.
         // Tiles wholly past n_kept hold evicted rows only: they store the
@@ -693,7 +771,8 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
         t_in = t_out = li < 0 ? 0u : ((uint32_t)li >= a.seq_in ? a.seq_in - 1u : (uint32_t)li);
         keep = t_raw < n_list;
         if (tile * 64u >= n_list) {
-            for (uint32_t j = j0; j < j1 && in_range; ++j) {
+            wide.init(nullptr, t_out, in_range);
+            for (uint32_t j = j0; j < j1; ++j) {
                 const uint32_t tensor = j % a.n_tensors;
                 RowOut o = {};
                 o.recon = tab_recon ? gptr<uint16_t>(tab_recon[tensor]) : nullptr;
@@ -701,7 +780,7 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
                 o.cosets = tab_cosets ? gptr<uint8_t>(tab_cosets[tensor]) : nullptr;
                 o.scales = tab_scales ? gptr<float>(tab_scales[tensor]) : nullptr;
                 const uint32_t bh = b * a.heads + j / a.n_tensors;
-                store_evicted_row<D, L, DR>(o, (size_t)bh * a.seq_out + t_out, q);
+                store_evicted_row<D, L, DR>(o, wide, bh * a.seq_out, t_out, q, in_range, a.stream_out != 0);
             }
             return;
         }
@@ -716,6 +795,10 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
     // rows this launch writes: all, or (soft eviction) only the kept / only the evicted ones
     const bool active = in_range && (a.keep_mode == NQ_KEEP_ZERO || keep == (a.keep_mode == NQ_KEEP_WRITE_KEPT));
     if (a.keep_mode != NQ_KEEP_ZERO) keep = true;  // selected rows are quantized as they are
+
+    __shared__ uint4 out_stage[WIDE ? 4 * 16 * (DR / 8) : 1];
+    if constexpr (WIDE)
+        wide.init(out_stage + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * (16 * (DR / 8)), t_out, active);
 
     // Keys: the RoPE rows of the source position, loaded once for the work item
     // (pages rotate at per-page positions, loaded per sub-item).
@@ -823,9 +906,9 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
             o.scales16 = nullptr;
         }
         if constexpr (HOLD_OUT)
-            quant_row_body<D, L, IS_KEY, DR, PAGE, GATHER>(a, x, cs, sn, co, so, q, o, bh, t_in, t_out, active, my_rope);
+            quant_row_body<D, L, IS_KEY, DR, PAGE, GATHER, WIDE>(a, wide, x, cs, sn, co, so, q, o, bh, t_in, t_out, active, my_rope);
         else
-            quant_row_body<D, L, IS_KEY, DR, PAGE, GATHER>(a, x, cs, sn, cs, sn, q, o, bh, t_in, t_out, active, my_rope);
+            quant_row_body<D, L, IS_KEY, DR, PAGE, GATHER, WIDE>(a, wide, x, cs, sn, cs, sn, q, o, bh, t_in, t_out, active, my_rope);
     }
 }
 

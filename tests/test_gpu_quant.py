@@ -409,3 +409,42 @@ def test_head_dim_96_values_equal_zero_padded_128_on_gpu():
         assert torch.equal(r96, r128[..., :96])
         assert torch.equal(c96.syms, c128.syms) and torch.equal(c96.scales, c128.scales)
         assert torch.equal(c96.cosets, c128.cosets)
+
+
+@pytest.mark.parametrize("d,key,n_t,shape,mode", [
+    (128, True, 20, (1, 7, 1003), "plain"), (128, False, 9, (2, 5, 1500), "list"),
+    (128, True, 13, (1, 8, 1500), "gather"), (96, False, 14, (1, 8, 1601), "plain"),
+    (256, True, 5, (1, 6, 2303), "list"), (64, True, 20, (1, 8, 1777), "soft"),
+])
+def test_large_launch_equals_single_tensor_launches(d, key, n_t, shape, mode):
+    """Launches of 32 MB and more store their reconstructions nontemporally: the
+    same bytes as one launch per tensor, which stays below that size."""
+    from nexusquant_amd import _lib
+    from nexusquant_amd.ops import quantize_tensors
+    print(f"[gpu] large launch d={d} key={key} {mode}", flush=True)
+    b, h, s = shape
+    g = torch.Generator(device=DEV).manual_seed(d + n_t)
+    xs = [torch.randn(b, h, s, d, generator=g, device=DEV).half() for _ in range(n_t)]
+    assert 2 * n_t * b * h * s * d * (0.9 if mode == "gather" else 1) >= 32 << 20 > 2 * b * h * s * d
+    kw = {}
+    if mode != "plain":
+        keep = torch.rand(b, s, generator=g, device=DEV) < 0.6
+        if mode == "gather":
+            kw["gather"] = torch.sort(torch.randperm(s, generator=g, device=DEV)[:int(0.95 * s)]).values.unsqueeze(0)
+        else:
+            kw["keep"] = keep.to(torch.uint8)
+        if mode == "list":
+            idx = [torch.cat([k.nonzero()[:, 0], (~k).nonzero()[:, 0].flip(0)]) for k in keep]
+            kw.update(order=torch.stack(idx).int(), n_kept=keep.sum(1).int())
+
+    def run(ts):
+        if mode != "soft":
+            return quantize_tensors(ts, is_key=key, levels=8, codes=True, **kw)[0]
+        out = [torch.zeros(b, h, s, d, dtype=torch.float16, device=DEV) for _ in ts]
+        for m, lv in ((_lib.NQ_KEEP_WRITE_KEPT, 8), (_lib.NQ_KEEP_WRITE_EVICTED, 2)):
+            quantize_tensors(ts, is_key=key, levels=lv, keep_mode=m, recon_out=out, **kw)
+        return out
+
+    many = run(xs)
+    for x, got in zip(xs, many):
+        assert torch.equal(got, run([x])[0])
