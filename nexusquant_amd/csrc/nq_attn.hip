@@ -7,13 +7,18 @@
 // the chunk's running max m, its sum of exp l and the unnormalised value sum
 // y.  A combine kernel merges the chunks of a row.
 //
-//  1. Keys, a quad of lanes per token (the page decoder's layout): exact
-//     fp16 Walsh-Hadamard of the integer codes without the top stage, one
-//     scale multiply, the merged top stage + forward RoPE at the stored
-//     position, rounding to fp16 -- bit for bit the keys the page decoder
-//     writes -- then q . k divided by fl(sqrt(head_dim)): a 16x16x32 fp16 MFMA
-//     per 32 coordinates for fp16 queries with 8 heads per kv head, else
-//     v_dot2_f32_f16 (fp16 queries) or fp32 FMAs.  Logits go to LDS.
+//  1. Keys on the matrix cores, 16 tokens (a unit) at a time.  A key is
+//     R(pos) H c scale h_D / 2 with c its int8 codes; the Walsh-Hadamard stages
+//     below the top one are the products of the two half rows of c with the +-1
+//     matrix of half the size: 16x16x64 int8 MFMAs, exact in int32, straight from
+//     the page's bytes (the codes are the B operand, 16 consecutive bytes a lane).
+//     A result tile leaves each lane 4 coordinates of its token, and of the
+//     coordinates D/2 further on: RoPE's pairs, so the merged top stage + forward
+//     RoPE is lane-local.  Rounded to fp16 the tiles are the A operand of
+//     16x16x32 MFMAs with the query heads as columns, their k order matched by the
+//     order the queries are laid out in LDS.  The row scale multiplies the logit, in
+//     fp32, not the key: one rounding per coordinate either way.  bf16 queries take
+//     the keys as two bf16 parts, fp32 queries fp32 FMAs on the unrounded keys.
 //  2. Per query head the chunk max x_m of the unscaled logits and
 //     e = exp((x - x_m) / scale_divisor), l = sum e (fixed order); LDS keeps
 //     the weight e * scale_v / 2 per token as an fp16 pair hi + lo.
@@ -23,6 +28,19 @@
 //     weights x codes over the chunk, 32 tokens per MFMA; the combine kernel
 //     weights the chunks' sums, applies S and h_D once per (row, query head)
 //     and divides by the softmax sum.
+//
+// What bounds it: the latency of a unit's loads and of the three phases one after
+// another; the vector ALUs are busy about half the time (3550 instructions a wave;
+// 4600 when the keys were decoded on them, a quad of lanes a token), the page bytes
+// move at 2.9 TB/s.  Measured against that form, call between events, us: 64/8 heads
+// x 131072 tokens 121.3 -> 116.5; 32/32 heads x 4 x 8192 100.7 -> 99.5; 32/8 bf16, 8
+// ragged rows up to 4096 40.0 -> 34.0, and 26.8 with the shorter chunks below.
+//
+// Chunks are 512 tokens when that makes enough workgroups, else shorter: the caller
+// halves them down to 64 tokens while chunks x kv heads is below two per CU (512).
+// 32/8 heads x 1000 tokens 27.2 -> 15.2 us, 32 ragged rows up to 600 31.9 -> 25.8; a
+// threshold of 1024 or 2048 is slower where the combine kernel then has more to add
+// (26.8 us at 512, 29.0 at 1024, 33.8 at 2048 on the eight ragged rows).
 //
 // Work items are (chunk, kv head) with the kv head fastest, and block 8k + x
 // takes item x * per_xcd + k: the kv heads of one chunk run on one XCD and
@@ -84,14 +102,6 @@ __device__ __forceinline__ UnitRec unit_rec(const AttnArgs& a, int u) {
     return x;
 }
 
-// int8 codes of one dword -> two exact fp16 pairs (see codes_to_f16 in nq_page.hip)
-__device__ __forceinline__ void attn_codes_f16(uint32_t w, half2v& lo, half2v& hi) {
-    const uint32_t u = w ^ 0x80808080u;
-    const half2v bias = {(__fp16)-1152.0f, (__fp16)-1152.0f};
-    lo = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(u, 0x64646464u, 0x00050004u)) + bias;
-    hi = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(u, 0x64646464u, 0x00070006u)) + bias;
-}
-
 template <int DT>
 __device__ __forceinline__ float attn_load_f32(const void* p, size_t i) {
     if constexpr (DT == NQ_F32) return static_cast<const float*>(p)[i];
@@ -102,6 +112,58 @@ __device__ __forceinline__ float attn_load_f32(const void* p, size_t i) {
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef int int4v __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(float2v{a, b}, bf16x2v));
+}
+
+// The half-row Walsh-Hadamard matrix as int8 MFMA A operands.  Rows are output
+// coordinates m = 16 t + r (r = lane % 16), columns the codes k = KB u + KPL kg + j
+// (kg = lane / 16, j the lane's byte): entry (-1)^popcount(m & k), which is the
+// entry of tile 0 and step 0 with its sign set by a parity of t, u and kg alone.
+template <int D>
+struct KeyMfma {
+    static constexpr int HALF = D / 2;
+    static constexpr int KB = HALF < 64 ? 32 : 64;  // codes per MFMA
+    static constexpr int KPL = KB / 4;              // of them per lane
+    static constexpr int NK = HALF / KB;            // MFMAs per tile
+    static constexpr int T = HALF / 16;             // tiles per half row
+    static constexpr int W = KPL / 4;               // operand dwords
+    uint32_t h[W];
+
+    __device__ __forceinline__ void init(int lane) {
+        const uint32_t r = lane & 15, kg = lane >> 4;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            uint32_t v = 0;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const uint32_t k = KPL * kg + 4 * w + b;
+                v |= (uint32_t)((__builtin_popcount(r & k & 15u) & 1) ? 0xff : 0x01) << (8 * b);
+            }
+            h[w] = v;
+        }
+    }
+    // acc += (tile t, step u) x the codes
+    __device__ __forceinline__ int4v mul(int t, int u, int lane, const uint32_t (&c)[W], int4v acc) const {
+        const uint32_t kg = lane >> 4;
+        const uint32_t hi = (KB == 64 ? 4u * u + kg : kg >> 1) & (uint32_t)t;  // the bits of k from 16 on
+        const uint32_t flip = (__builtin_popcount(hi) & 1) ? 0xfefefefeu : 0u; // +1 <-> -1
+        if constexpr (KB == 64) {
+            const int4v a = {(int)(h[0] ^ flip), (int)(h[1] ^ flip), (int)(h[2] ^ flip), (int)(h[3] ^ flip)};
+            const int4v b = {(int)c[0], (int)c[1], (int)c[2], (int)c[3]};
+            return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, acc, 0, 0, 0);
+        } else {
+            const uint64_t a = (uint64_t)(h[0] ^ flip) | (uint64_t)(h[1] ^ flip) << 32;
+            const uint64_t b = (uint64_t)c[0] | (uint64_t)c[1] << 32;
+            return __builtin_amdgcn_mfma_i32_16x16x32_i8((long)a, (long)b, acc, 0, 0, 0);
+        }
+    }
+};
 
 // wave-wide reductions (64 lanes) through LDS-free cross-lane moves
 __device__ __forceinline__ float wave_max(float v) {
@@ -115,21 +177,32 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-template <int D, int G, int QDT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 4 : 2))) void paged_attn_kernel(
+// MT: the merged RoPE tables are given (else they are formed from cos and sin;
+// a template, because a branch between an MFMA and the first use of its result
+// hides the wait that the result needs from the compiler's hazard checks).
+// Registers: fp16 queries fit 4 waves per SIMD at D = 128 (121 VGPRs), the others
+// would spill there and take 3, fp32 queries of 4 heads 2.
+template <int D, int G, int QDT, bool MT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : D == 256 || (QDT == NQ_F32 && G >= 4) ? 2 : QDT == NQ_F16 ? 4 : 3))) void paged_attn_kernel(
     AttnArgs a) {
-    constexpr int C = D / 32;
+    using KM = KeyMfma<D>;
     constexpr bool QF16 = QDT == NQ_F16;
+    constexpr bool QF32 = QDT == NQ_F32;
+    // the queries: MFMA operands [tile][lane], or for fp32 [head][tile][kg] x 8 floats
+    constexpr int QOP = QF32 ? G * KM::T * 4 * 2 : KM::T * 64;
     __shared__ __attribute__((aligned(16))) float s_w[kChunk * G];  // [token][head]: logits, then e * scale_v / 2
     __shared__ float s_a[kChunk];       // scale_v / 2 per token
+    __shared__ float s_k[kChunk];       // scale_k h_D / 2 per token
     __shared__ float s_red[4][G];   // per wave: each head's max, then
     __shared__ float s_sum[4][G];   // its sum of exp
-    __shared__ float s_acc[4][G][D];
+    // the query operands until the logits are done, then the waves' value sums
+    __shared__ uint4 s_buf[QOP > 4 * G * D / 4 ? QOP : 4 * G * D / 4];
+    uint4* const s_q = s_buf;
+    float (*const s_acc)[G][D] = reinterpret_cast<float (*)[G][D]>(s_buf);
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int q = lane & 3;
-    const int quad = lane >> 2;
+    const int n16 = lane & 15, kg = lane >> 4;
     const uint32_t w_item = (blockIdx.x & 7u) * a.per_xcd + (blockIdx.x >> 3);
     if (w_item >= a.work) return;  // whole block
     const uint32_t chunk = w_item / a.kv_heads;
@@ -138,147 +211,190 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 
     const int u0 = a.chunk_units[chunk], u1 = a.chunk_units[chunk + 1];
     const int n_tok = a.chunk_tokens[chunk] < kChunk ? a.chunk_tokens[chunk] : kChunk;
 
-    // the G query heads of this kv head in LDS (fp16 queries as fp16, others as
-    // fp32); every quad reads the same slices, so the reads are broadcasts
-    using qreg_t = typename std::conditional<QF16, half2v, float>::type;
-    constexpr int QR = QF16 ? 4 : 8;  // registers per 8 coordinates
-    __shared__ __attribute__((aligned(16))) qreg_t s_q[G][C][4][QR];
-    for (int i = threadIdx.x; i < G * D; i += 256) {
-        const int g = i / D, j = i % D;
-        const size_t qi = ((size_t)row * a.q_heads + kh * G + g) * D + j;
-        const int c = j / 32, qq = (j / 8) % 4, k = j % 8;
-        if constexpr (QF16) {
-            reinterpret_cast<uint16_t*>(&s_q[g][c][qq][0])[k] = static_cast<const uint16_t*>(a.query)[qi];
-        } else {
-            s_q[g][c][qq][k] = attn_load_f32<QDT>(a.query, qi);
+    // the query heads in the order the keys come out: block (t, kg) holds the
+    // coordinates 16 t + 4 kg + 0..3 and those D / 2 on.  As MFMA operands lane l of
+    // tile t holds head l % 16 (zero past G) and block l / 16.
+    const size_t q_base = ((size_t)row * a.q_heads + kh * G) * D;
+    if constexpr (QF32) {
+        float* const sq = reinterpret_cast<float*>(s_q);
+        for (int i = threadIdx.x; i < G * D; i += 256) {
+            const int n = i / D, r = i % D, t = r >> 5, g4 = (r >> 3) & 3, e = r & 7;
+            sq[i] = static_cast<const float*>(a.query)[q_base + (size_t)n * D + 16 * t + 4 * g4 + (e & 3) + (e >> 2) * KM::HALF];
         }
-    }
-    __syncthreads();
-    const float qsig = quad_sign(q);
-
-    // fp16 queries with 8 heads per kv head take q . k on the matrix cores: per
-    // unit and chunk c one 16x16x32 fp16 MFMA with the unit's 16 keys as the A
-    // rows and the query heads as the B columns (heads 8..15 zero).  Lane l
-    // holds B for head l % 16 over coordinates 32c + 8 (l / 16) .. + 7.
-    constexpr bool QK_MFMA = QF16 && G == 8;
-    half8v qb[QK_MFMA ? C : 1];
-    if constexpr (QK_MFMA) {
-        const int n = lane & 15, kg = lane >> 4;
+    } else {
+        for (int i = threadIdx.x; i < KM::T * 64; i += 256) {
+            const int t = i >> 6, n = i & 15, g4 = (i >> 4) & 3;
+            uint32_t v[4] = {};
+            if (n < G) {
+                const uint16_t* qp = static_cast<const uint16_t*>(a.query) + q_base + (size_t)n * D + 16 * t + 4 * g4;
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const uint4 v = n < G ? *reinterpret_cast<const uint4*>(&s_q[n][c][kg][0]) : make_uint4(0u, 0u, 0u, 0u);
-            qb[c] = __builtin_bit_cast(half8v, v);
+                for (int k = 0; k < 4; ++k) {
+                    const int at = (k >> 1) * KM::HALF + 2 * (k & 1);
+                    v[k] = (uint32_t)qp[at] | (uint32_t)qp[at + 1] << 16;
+                }
+            }
+            s_q[i] = make_uint4(v[0], v[1], v[2], v[3]);
         }
     }
+    KM km;
+    km.init(lane);
+    __syncthreads();
 
-    // ---- 1. keys and logits, one token per quad, 16 tokens per unit ----
+    // ---- 1. keys and logits, 16 tokens per unit ----
     // The next unit's record and key codes are loaded while the current one is
     // decoded (indices clamped, so every load is unconditional and in bounds).
+    // The MFMA operands want token n16 and 16-byte block kg in lane 16 kg + n16,
+    // where a load instruction's neighbouring lanes would each touch another cache
+    // line.  Codes and table rows are therefore loaded a quad per token, 64
+    // consecutive bytes, and moved to their lanes by ds_bpermute (64 query heads, 8
+    // kv heads, 131072 tokens, between events: 131 us loaded in place, 121 so).
     struct KeyIn {
-        uint2 w[C];
+        uint32_t c[2][KM::NK][KM::W];
         uint32_t ks, vs;
-        int32_t pos;
     };
+    const int q = lane & 3, quad = lane >> 2;
+    const int from_quad = 4 * (4 * n16 + kg);  // byte address of the lane that loaded this lane's block
     auto load_keys = [&](const UnitRec& r, KeyIn& k) {
         const int t = quad < r.n ? quad : 0;
-        const size_t row = (size_t)kh * r.stride + t;
-        const int8_t* crow = r.kc + row * D;
+        const int8_t* p = r.kc + ((size_t)kh * r.stride + t) * D + KM::KPL * q;
 #pragma unroll
-        for (int c = 0; c < C; ++c) k.w[c] = *reinterpret_cast<const uint2*>(crow + 32 * c + 8 * q);
-        k.ks = r.ks[row];
-        k.vs = r.vs[row];
-        k.pos = r.pos[t];
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int u = 0; u < KM::NK; ++u) {
+                const uint32_t* w = reinterpret_cast<const uint32_t*>(p + hf * KM::HALF + u * KM::KB);
+#pragma unroll
+                for (int i = 0; i < KM::W; ++i) k.c[hf][u][i] = w[i];
+            }
+        const size_t srow = (size_t)kh * r.stride + (n16 < r.n ? n16 : 0);
+        k.ks = r.ks[srow];
+        k.vs = r.vs[srow];
     };
+    auto load_pos = [&](const UnitRec& r) {
+        const int32_t p = r.pos[quad < r.n ? quad : 0];
+        return p;
+    };
+    // The token's table rows, 16 t + 4 q .. of each: a tile's pair is loaded for the
+    // next unit as soon as the current unit's is used, into the same registers.
+    const float* const tab0 = MT ? a.rope_dm : a.rope_cos;
+    const float* const tab1 = MT ? a.rope_dp : a.rope_sin;
+    float4v dm[KM::T], dp[KM::T];
+    auto tab_row = [&](int32_t p) {
+        const uint32_t pos = p < 0 ? 0u : ((uint32_t)p >= a.rope_n_pos ? a.rope_n_pos - 1u : (uint32_t)p);
+        return (size_t)pos * (D / 2) + 4 * q;
+    };
+    auto load_tables = [&](size_t row, int t) {
+        dm[t] = *reinterpret_cast<const float4v*>(tab0 + row + 16 * t);
+        dp[t] = *reinterpret_cast<const float4v*>(tab1 + row + 16 * t);
+    };
+    auto permute = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_bpermute(from_quad, (int)v); };
+    auto permute_f = [&](float v) { return __builtin_bit_cast(float, permute(__builtin_bit_cast(uint32_t, v))); };
     int u = u0 + wave;
-    UnitRec rc = unit_rec(a, u < u1 ? u : u0);
+    auto clampu = [&](int x) { return x < u1 ? x : (u < u1 ? u : u0); };
+    UnitRec rc = unit_rec(a, clampu(u)), rn = unit_rec(a, clampu(u + 4));
     KeyIn kin;
     load_keys(rc, kin);
+    {
+        const size_t row = tab_row(load_pos(rc));
+#pragma unroll
+        for (int t = 0; t < KM::T; ++t) load_tables(row, t);
+    }
+    int32_t pos_n = load_pos(rn);
     for (; u < u1; u += 4) {
-        const int un = u + 4 < u1 ? u + 4 : u;
-        const UnitRec rn = unit_rec(a, un);
+        const UnitRec r2 = unit_rec(a, clampu(u + 8));
         KeyIn knext;
         load_keys(rn, knext);
-
-        const int t = quad;
-        const bool valid = t < rc.n && rc.coff + t < kChunk;
-        half2v h[C][4];
+        const size_t row_n = tab_row(pos_n);
+        pos_n = load_pos(r2);
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            attn_codes_f16(kin.w[c].x, h[c][0], h[c][1]);
-            attn_codes_f16(kin.w[c].y, h[c][2], h[c][3]);
-        }
-        const float g = qsig * ((0.5f * f16_bits_to_f32(kin.ks)) * a.hscale);
-        const uint32_t pos = kin.pos < 0 ? 0u : ((uint32_t)kin.pos >= a.rope_n_pos ? a.rope_n_pos - 1u : (uint32_t)kin.pos);
-        float dm[C / 2][8], dp[C / 2][8];
-        load_rope_merged<D>(a.rope_cos, a.rope_sin, a.rope_dm, a.rope_dp, pos, q, dm, dp);
-        fwht_row_f16<C, false>(h, q);
-        float x[C][8];
+        for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-        for (int c = 0; c < C; ++c)
+            for (int s = 0; s < KM::NK; ++s)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                x[c][2 * k] = __builtin_fmaf((float)h[c][k].x, g, 0.0f);
-                x[c][2 * k + 1] = __builtin_fmaf((float)h[c][k].y, g, 0.0f);
+                for (int i = 0; i < KM::W; ++i) kin.c[hf][s][i] = permute(kin.c[hf][s][i]);
+        float4v la[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};  // two independent chains
+        float lf[QF32 ? G : 1] = {};
+#pragma unroll
+        for (int t = 0; t < KM::T; ++t) {
+            int4v y0 = {0, 0, 0, 0}, y1 = {0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < KM::NK; ++s) {
+                y0 = km.mul(t, s, lane, kin.c[0][s], y0);
+                y1 = km.mul(t, s, lane, kin.c[1][s], y1);
             }
-        rope_stage_merged<C>(x, dm, dp);
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) asm("" : "+v"(x[c][i]));  // fp32, then fp16: two roundings
-        half2v kf[C][4];
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) kf[c][k] = half2v{(__fp16)x[c][2 * k], (__fp16)x[c][2 * k + 1]};
-
-        if constexpr (QK_MFMA) {
-            // keys to the MFMA A layout: lane 16g + t takes token t's coordinates
-            // 32c + 8g .. + 7 from lane 4t + g (the quad layout)
-            const int addr_in = 4 * (4 * (lane & 15) + (lane >> 4));
-            float4v lg = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-                u32x4v bw;
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    bw[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(addr_in, (int)__builtin_bit_cast(uint32_t, kf[c][k]));
-                lg = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, bw), qb[c], lg, 0, 0, 0);
-            }
-            // lane l holds the logits of tokens 4 (l / 16) + i for head l % 16
-            const int n = lane & 15;
+            float m[4], p[4];  // fl(sin - cos), fl(cos + sin) of coordinates 16 t + 4 kg + i
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int tt = 4 * (lane >> 4) + i;
-                const float v = lg[i];
-                if (n < G && tt < rc.n && rc.coff + tt < kChunk) s_w[(rc.coff + tt) * G + n] = v;
+                m[i] = permute_f(dm[t][i]);
+                p[i] = permute_f(dp[t][i]);
             }
-        } else {
+            load_tables(row_n, t);
+            if constexpr (!MT) {
 #pragma unroll
-            for (int gq = 0; gq < G; ++gq) {
-                float acc = 0.0f;
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    qreg_t qv[QR];
-#pragma unroll
-                    for (int k = 0; k < QR; ++k) qv[k] = s_q[gq][c][q][k];
-                    if constexpr (QF16) {
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) acc = __builtin_amdgcn_fdot2(kf[c][k], qv[k], acc, false);
-                    } else {
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            acc = __builtin_fmaf((float)kf[c][k].x, qv[2 * k], acc);
-                            acc = __builtin_fmaf((float)kf[c][k].y, qv[2 * k + 1], acc);
-                        }
-                    }
+                for (int i = 0; i < 4; ++i) {
+                    const float cs = m[i], sn = p[i];
+                    m[i] = sn - cs;
+                    p[i] = cs + sn;
                 }
-                acc += dpp_f32<kQuadXor1>(acc);
-                acc += dpp_f32<kQuadXor2>(acc);
-                if (valid && q == 0) s_w[(rc.coff + t) * G + gq] = acc;
+            }
+            float x[8];  // coordinates 16 t + 4 kg + i, and those D / 2 on
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float lo = (float)y0[i], hi = (float)y1[i];
+                x[i] = __builtin_fmaf(-lo, m[i], hi * p[i]);
+                x[4 + i] = __builtin_fmaf(lo, p[i], hi * m[i]);
+            }
+            if constexpr (QF16) {
+                u32x4v kf;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) asm("" : "+v"(x[i]));  // one packed conversion per pair, not two mixed fmas
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    kf[k] = __builtin_bit_cast(uint32_t, half2v{(__fp16)x[2 * k], (__fp16)x[2 * k + 1]});
+                la[t & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, kf),
+                                                                   __builtin_bit_cast(half8v, s_q[t * 64 + lane]), la[t & 1], 0, 0, 0);
+            } else if constexpr (QDT == NQ_BF16) {
+                u32x4v kp[2];  // the key as two bf16 parts
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    kp[0][k] = pk_bf16(x[2 * k], x[2 * k + 1]);
+                    kp[1][k] = pk_bf16(x[2 * k] - __builtin_bit_cast(float, kp[0][k] << 16),
+                                       x[2 * k + 1] - __builtin_bit_cast(float, kp[0][k] & 0xffff0000u));
+                }
+                const bf16x8v qv = __builtin_bit_cast(bf16x8v, s_q[t * 64 + lane]);
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    la[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, kp[k]), qv, la[k], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const float* qv = reinterpret_cast<const float*>(s_q) + g * D + 32 * t + 8 * kg;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) lf[g] = __builtin_fmaf(x[i], qv[i], lf[g]);
+                }
             }
         }
-        if (valid && q == 1) s_a[rc.coff + t] = 0.5f * f16_bits_to_f32(kin.vs);
+        if constexpr (QF32) {  // each lane has its 32 coordinates' part of token n16's logits
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                lf[g] += __shfl_xor(lf[g], 16, 64);
+                lf[g] += __shfl_xor(lf[g], 32, 64);
+                if (kg == 0 && n16 < rc.n && rc.coff + n16 < kChunk) s_w[(rc.coff + n16) * G + g] = lf[g];
+            }
+        } else {
+            // lane l holds the logits of tokens 4 (l / 16) + i for head l % 16
+            const float4v lg = la[0] + la[1];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int tt = 4 * kg + i;
+                if (n16 < G && tt < rc.n && rc.coff + tt < kChunk) s_w[(rc.coff + tt) * G + n16] = lg[i];
+            }
+        }
+        if (kg == 0 && n16 < rc.n && rc.coff + n16 < kChunk) {
+            s_a[rc.coff + n16] = 0.5f * f16_bits_to_f32(kin.vs);
+            s_k[rc.coff + n16] = (0.5f * f16_bits_to_f32(kin.ks)) * a.hscale;
+        }
         rc = rn;
+        rn = r2;
         kin = knext;
     }
     __syncthreads();
@@ -290,7 +406,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 
     __shared__ float s_amax[4];
     {
         float v = -__builtin_inff();
-        for (int i = threadIdx.x; i < n_tok * G; i += 256) v = __builtin_fmaxf(v, s_w[i]);
+        for (int i = threadIdx.x; i < n_tok * G; i += 256) {
+            const float x = s_w[i] * s_k[i / G];  // read again by this thread below
+            s_w[i] = x;
+            v = __builtin_fmaxf(v, x);
+        }
 #pragma unroll
         for (int o = 32; o >= G; o >>= 1) v = __builtin_fmaxf(v, __shfl_xor(v, o, 64));
         if (lane < G) s_red[wave][lane] = v;
@@ -342,9 +462,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 
     constexpr int NB = D / 16;
     using cword_t = typename std::conditional<NB == 4, uint32_t,
                                               typename std::conditional<NB == 8, uint2, uint4>::type>::type;
-    const int n16 = lane & 15, kg = lane >> 4;
     const bool second = kg >= 2;
-    const int tb = 8 * (kg & 1);
+    const int tok0 = 8 * (kg & 1);
     const bool has_w = n16 < 2 * G;
     const int w_half = 2 * (n16 % G) + (n16 >= G ? 1 : 0);  // fp16 index within a token's G hi/lo pairs
     const _Float16* s_wh = reinterpret_cast<const _Float16*>(s_w);
@@ -372,7 +491,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 
         const int8_t* base = r.vc + (size_t)kh * r.stride * D + NB * n16;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const int t = tb + s < r.n ? tb + s : r.n - 1;
+            const int t = tok0 + s < r.n ? tok0 + s : r.n - 1;
             const cword_t x = *reinterpret_cast<const cword_t*>(base + (size_t)t * D);
             const uint32_t* xw = reinterpret_cast<const uint32_t*>(&x);
 #pragma unroll
@@ -395,8 +514,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 
         half8v wa;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const bool ok = has_w && tb + s < vr.nw;
-            const _Float16 w = s_wh[ok ? 2 * G * (vr.coff + tb + s) + w_half : 0];
+            const bool ok = has_w && tok0 + s < vr.nw;
+            const _Float16 w = s_wh[ok ? 2 * G * (vr.coff + tok0 + s) + w_half : 0];
             wa[s] = ok ? w : (_Float16)0.0f;
         }
 #pragma unroll
@@ -541,7 +660,8 @@ __global__ __launch_bounds__(1024) void paged_attn_combine(AttnArgs a) {
 template <int D, int G, int QDT>
 static hipError_t launch_attn(const AttnArgs& a, uint32_t n_chunks, uint32_t batch, hipStream_t s) {
     if (n_chunks > 0) {
-        hipLaunchKernelGGL((paged_attn_kernel<D, G, QDT>), dim3(a.per_xcd * 8u), dim3(256), 0, s, a);
+        if (a.rope_dm) hipLaunchKernelGGL((paged_attn_kernel<D, G, QDT, true>), dim3(a.per_xcd * 8u), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((paged_attn_kernel<D, G, QDT, false>), dim3(a.per_xcd * 8u), dim3(256), 0, s, a);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -330,6 +330,30 @@ class NexusQuantKVCompressor:
 # Decode attention over compressed pages
 # ---------------------------------------------------------------------------
 
+# Workgroups (chunk, kv head) a plan should have before its chunks stay at the
+# kernel's full length: two per CU.  32 query / 8 kv heads x 1000 tokens: 27 us with
+# 512-token chunks, 15 with 64; a threshold of 1024 cost 2 us on ragged batches of 8
+# and 32 rows, whose combine pass then adds twice the chunks.
+_MIN_WORKGROUPS = 512
+_MIN_CHUNK = 64  # one 16-token unit for each of a workgroup's four waves
+
+
+def _tokens_used(row: Sequence[Tuple[int, int]], ctx: int) -> int:
+    """Tokens a row attends to: the first ctx of its pages' tokens (a Python slice's
+    semantics: a negative length drops tokens from the end, 0 none)."""
+    avail = sum(n for _, n in row)
+    use = 0 if ctx == 0 else (ctx if ctx > 0 else avail + ctx)
+    return max(0, min(use, avail))
+
+
+def chunk_length(used: Sequence[int], kv_heads: int, cap: int) -> int:
+    """Chunk length for rows of `used` tokens: cap, halved while the plan would have
+    fewer than _MIN_WORKGROUPS workgroups and a half still is _MIN_CHUNK tokens."""
+    while cap >= 2 * _MIN_CHUNK and sum(-(-n // cap) for n in used) * kv_heads < _MIN_WORKGROUPS:
+        cap //= 2
+    return cap
+
+
 def build_chunk_plan(rows: Sequence[Sequence[Tuple[int, int]]], context_lens: Sequence[int], chunk_cap: int):
     """Cut each row's token stream into chunks of at most chunk_cap tokens.
 
@@ -347,10 +371,7 @@ def build_chunk_plan(rows: Sequence[Sequence[Tuple[int, int]]], context_lens: Se
     row_chunks = [0]
     total = 0
     for b, row in enumerate(rows):
-        ctx = int(context_lens[b])
-        avail = sum(n for _, n in row)
-        use = 0 if ctx == 0 else (ctx if ctx > 0 else avail + ctx)
-        use = max(0, min(use, avail))
+        use = _tokens_used(row, int(context_lens[b]))
         fill = None  # tokens in the row's open chunk (None: none open)
         for slot, n_page in row:
             if use == 0:
@@ -501,6 +522,8 @@ class NexusQuantPagedAttention:
                         slot_pages.append(p)
                     row.append((slot_of[id(p)], p.key_codes.shape[1]))
             rows.append(row)
+        used = [_tokens_used(row, c) for row, c in zip(rows, ctx)]
+        chunk_cap = chunk_length(used, kv_heads or 1, chunk_cap)
         parts, total = build_chunk_plan(rows, ctx, chunk_cap)
         n_chunks = len(parts["chunk_row"])
         dev = None

@@ -331,3 +331,42 @@ def test_compress_and_cache_follows_reference_semantics():
         assert torch.equal(page.positions.cpu(), pos)
         mism = (page.key_codes.cpu().reshape(-1, 8) != kc.reshape(-1, 8)).any(1).float().mean().item()
         assert mism <= 2e-2
+
+
+@pytest.mark.parametrize("d,group,qdt", [(64, 8, torch.float16), (128, 8, torch.float16), (128, 1, torch.bfloat16),
+                                         (128, 4, torch.float32), (256, 2, torch.float32), (256, 4, torch.bfloat16)])
+@pytest.mark.parametrize("ctx", [1, 15, 17, 63, 65, 128, 129, 1000])
+def test_paged_forward_short_contexts_and_table_kinds(d, group, qdt, ctx):
+    """Contexts around a unit (16 tokens) and the shortest chunk (64), where some of a
+    workgroup's waves have no unit: against float64 attention over the decoded pages,
+    and the same bits from cos / sin tables as from the merged ones."""
+    from nexusquant_amd.vllm_backend import CompressedPage, NexusQuantKVCompressor, NexusQuantPagedAttention
+    print(f"[gpu] short context d={d} group={group} {qdt} ctx={ctx}", flush=True)
+    kv, block = 2, 16
+    g = torch.Generator(device=DEV).manual_seed(d + group + ctx)
+    comp = NexusQuantKVCompressor(head_dim=d, bits=3, rope_base=10000.0)
+    attn = NexusQuantPagedAttention(comp)
+    n_pages = -(-ctx // block)
+    cache = {}
+    for i in range(n_pages):
+        k = torch.randn(kv, block, d, device=DEV, generator=g).half()
+        v = (torch.randn(kv, block, d, device=DEV, generator=g) * 0.5).half()
+        cache[i] = comp.compress_page(k, v, torch.arange(i * block, (i + 1) * block, dtype=torch.int32) + 70000)
+    q = torch.randn(1, kv * group, d, device=DEV, generator=g).to(qdt)
+    plan = attn.plan(cache, [list(range(n_pages))], [ctx])
+    got = attn.run(plan, q)
+    tables = comp._tables
+    comp._tables = lambda m, dev: tables(m, dev)[:2] + (None, None)
+    assert torch.equal(attn.run(plan, q), got)
+    comp._tables = tables
+    dec = comp.decompress_pages([cache[i] for i in range(n_pages)])
+    k = torch.cat([p[0] for p in dec], 1)[:, :ctx].double()
+    v = torch.cat([p[1] for p in dec], 1)[:, :ctx].double()
+    want = torch.empty(1, kv * group, d, dtype=torch.float64, device=DEV)
+    for h in range(kv * group):
+        w = torch.softmax(k[h // group] @ q[0, h].double() / math.sqrt(d), 0)
+        want[0, h] = w @ v[h // group]
+    # _close_fp16's bounds are for a reference rounded as the op rounds: to fp16, then the
+    # query's type (an unrounded one alone is up to 2^-8 from a bf16 output)
+    want = want.half().to(qdt)
+    _close_fp16(got.float().cpu().numpy(), want.float().cpu().numpy(), bf16=qdt == torch.bfloat16)

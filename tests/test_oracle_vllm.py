@@ -154,3 +154,14 @@ def test_chunk_plan_walks_the_reference_token_order():
                 assert seen.all()
                 got[-ct[c]:] = sorted(got[-ct[c]:])
             assert [(s, t) for _, s, t in got] == want[b]
+
+
+@pytest.mark.parametrize("used,kv,cap,want", [
+    ([131072], 8, 512, 512), ([32768], 8, 512, 512), ([32767], 8, 512, 512), ([32256], 8, 512, 256),
+    ([4096] * 8, 8, 512, 512), ([4096] * 4, 8, 512, 256), ([1000], 8, 512, 64), ([], 1, 512, 64), ([0, 5], 32, 512, 64),
+    ([70] * 300, 2, 512, 512), ([10 ** 6], 1, 64, 64), ([10], 1, 16, 16),
+])
+def test_chunk_length_rule(used, kv, cap, want):
+    """Full-length chunks from two workgroups a CU on, else halves down to 64 tokens."""
+    from nexusquant_amd.vllm_backend import chunk_length
+    assert chunk_length(used, kv, cap) == want
