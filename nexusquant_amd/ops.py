@@ -60,6 +60,7 @@ class _AddressRing:
         self.host = torch.empty(self.ENTRIES, dtype=torch.int64, pin_memory=True)
         self.host_np = self.host.numpy()
         self.dev = torch.empty(self.ENTRIES, dtype=torch.int64, device=device)
+        self.host_addr, self.dev_addr = self.host.data_ptr(), self.dev.data_ptr()
         self.head = 0
         self.busy: List[Tuple[int, int, torch.cuda.Event]] = []  # oldest first
         # The runtime creates an event's resources at its first record, which can
@@ -85,7 +86,8 @@ class _AddressRing:
                 keep.append((s0, e0, ev))
         self.busy = keep
 
-    def stage(self, flat: List[int]) -> Tuple[torch.Tensor, Tuple[int, int]]:
+    def stage(self, flat: List[int]) -> Tuple[int, Tuple[int, int]]:
+        """The device address of the staged span (copied on the current stream), and the span."""
         n = len(flat)
         if n > self.ENTRIES:
             raise ValueError(f"{n} tensors in one launch exceed the address ring ({self.ENTRIES})")
@@ -94,9 +96,11 @@ class _AddressRing:
             end = start + n
             self._wait_for(start, end)
             self.host_np[start:end] = flat
-            self.dev[start:end].copy_(self.host[start:end], non_blocking=True)
+            with torch.cuda.device(self.device):
+                _lib.copy_to_device_async(self.dev_addr + 8 * start, self.host_addr + 8 * start, 8 * n,
+                                          _lib.current_stream_handle(self.device))
             self.head = end
-        return self.dev[start:end], (start, end)
+        return self.dev_addr + 8 * start, (start, end)
 
     def release(self, span: Tuple[int, int]) -> None:
         with self.lock:
@@ -123,9 +127,9 @@ def _ring(device) -> _AddressRing:
 
 
 class _PtrArrays:
-    """Device int64 arrays of the base addresses of each tensor group, staged
-    through the device's address ring.  Call release() right after the launch
-    that reads them."""
+    """Device addresses of int64 arrays of the base addresses of each tensor
+    group, staged through the device's address ring.  Call release() right after
+    the launch that reads them."""
 
     def __init__(self, groups: Sequence[Optional[Sequence[torch.Tensor]]], device):
         flat: List[int] = []
@@ -143,7 +147,7 @@ class _PtrArrays:
             return
         self._ring = _ring(device)
         dev, self._span = self._ring.stage(flat)
-        self.arrays = [None if sp is None else dev[sp[0]:sp[0] + sp[1]] for sp in spans]
+        self.arrays = [None if sp is None else dev + 8 * sp[0] for sp in spans]
 
     def release(self) -> None:
         if self._ring is not None and self._span is not None:
@@ -151,8 +155,11 @@ class _PtrArrays:
             self._span = None
 
 
-def _addr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+def _addr(t):
+    """A tensor's, or a staged array's, address as a pointer argument."""
+    if t is None:
+        return None
+    return ctypes.c_void_p(t if isinstance(t, int) else t.data_ptr())
 
 
 _workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
@@ -183,13 +190,21 @@ def release_workspaces() -> None:
         _workspaces.clear()
 
 
+def _check_gather(g: torch.Tensor, s: int) -> None:
+    """Raise unless every gather index lies in [0, s) (reads the list back: one round trip)."""
+    if g.numel():
+        lo, hi = torch.stack(torch.aminmax(g)).tolist()
+        if lo < 0 or hi >= s:
+            raise ValueError(f"gather indices must lie in [0, {s})")
+
+
 def quantize_tensors(tensors: Sequence[torch.Tensor], *, is_key: bool, levels: int,
                      rope_base: float = 10000.0, rope_scaling: Optional[dict] = None,
                      gather: Optional[torch.Tensor] = None, keep: Optional[torch.Tensor] = None,
                      keep_mode: int = _lib.NQ_KEEP_ZERO, recon_out: Optional[Sequence[torch.Tensor]] = None,
                      recon: bool = True, codes: bool = False, launch_events=None, merged_tables: bool = True,
                      order: Optional[torch.Tensor] = None, n_kept: Optional[torch.Tensor] = None,
-                     ) -> Tuple[Optional[List[torch.Tensor]], Optional[List[PackedCodes]]]:
+                     gather_checked: bool = False) -> Tuple[Optional[List[torch.Tensor]], Optional[List[PackedCodes]]]:
     """Run the fused quantizer over same-shaped [b, h, s, d] tensors in one launch.
 
     gather: int32/int64 [b, seq_out] source token per output row (truncation).
@@ -206,6 +221,8 @@ def quantize_tensors(tensors: Sequence[torch.Tensor], *, is_key: bool, levels: i
             the evicted ones) and n_kept [b], with `keep` and keep_mode
             NQ_KEEP_ZERO: only the kept rows are read and quantized; evicted rows
             get the zero-row outputs directly.  Same results as without them.
+    gather_checked: the caller knows the gather indices to lie in [0, seq_in)
+            (keep_mask's own list), so they are not read back to be checked.
     Returns (fp16 reconstructions or None, PackedCodes or None), one per tensor.
     """
     lib = _lib.load()
@@ -237,8 +254,8 @@ def quantize_tensors(tensors: Sequence[torch.Tensor], *, is_key: bool, levels: i
         if g.shape[0] != b:
             raise ValueError(f"gather must be [batch, seq_out], got {tuple(g.shape)}")
         seq_out = g.shape[1]
-        if g.numel() and (int(g.min()) < 0 or int(g.max()) >= s):
-            raise ValueError(f"gather indices must lie in [0, {s})")
+        if not gather_checked:
+            _check_gather(g, s)
     k = None
     if keep is not None:
         k = keep.to(device=dev, dtype=torch.uint8).contiguous()
@@ -467,8 +484,9 @@ def merge_values(values: Sequence[torch.Tensor], keep: torch.Tensor, kept_idx: t
 
 
 def gather_rows(tensors: Sequence[torch.Tensor], *, gather: Optional[torch.Tensor] = None,
-                keep: Optional[torch.Tensor] = None) -> List[torch.Tensor]:
-    """fp16 passthrough of same-shaped tensors: gathered rows or zeroed evicted rows."""
+                keep: Optional[torch.Tensor] = None, gather_checked: bool = False) -> List[torch.Tensor]:
+    """fp16 passthrough of same-shaped tensors: gathered rows or zeroed evicted rows
+    (gather_checked: as for quantize_tensors)."""
     lib = _lib.load()
     if not tensors:
         return []
@@ -485,8 +503,8 @@ def gather_rows(tensors: Sequence[torch.Tensor], *, gather: Optional[torch.Tenso
         if g.dim() == 1:
             g = g.unsqueeze(0).expand(b, -1).contiguous()
         seq_out = g.shape[1]
-        if g.numel() and (int(g.min()) < 0 or int(g.max()) >= s):
-            raise ValueError(f"gather indices must lie in [0, {s})")
+        if not gather_checked:
+            _check_gather(g, s)
     k = None
     if keep is not None:
         k = keep.to(device=dev, dtype=torch.uint8).contiguous()

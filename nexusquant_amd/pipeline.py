@@ -311,10 +311,11 @@ class NexusQuantEvict:
             return self._score_importance_real(model, input_ids), k_score
         return self._score_importance(k_score), k_score
 
-    def _apply(self, past_key_values, n_layers: int, skip: set, *, keep=None, gather=None, soft=False,
+    def _apply(self, past_key_values, n_layers: int, skip: set, *, keep=None, gather=None, seq=0, soft=False,
                kept_idx=None, n_kept=None):
         """Quantize (or pass through at fp16) every layer with one mask / gather list.
 
+        gather: positions of keep_mask's list, so inside [0, seq).
         soft: kept rows at the layer's levels and evicted rows at levels 2, no row
         zeroed (pipeline.py:1129-1183); protected layers pass through unmasked.
         kept_idx / n_kept (keep_mask's row list): mask eviction reads and
@@ -337,7 +338,8 @@ class NexusQuantEvict:
             kp = None if keep is None else keep[:, :s_l]
             gp = None
             if gather is not None:
-                gp = gather[gather < s_l].unsqueeze(0)
+                # the list covers the scored layer's positions: only a shorter layer drops some
+                gp = (gather if s_l >= seq else gather[gather < s_l]).unsqueeze(0)
             return kp, gp
 
         for key, layers in passthrough.items():
@@ -346,8 +348,8 @@ class NexusQuantEvict:
                 kp = None
             ks = [get_layer_kv(past_key_values, li)[0] for li in layers]
             vs = [get_layer_kv(past_key_values, li)[1] for li in layers]
-            k_out = gather_rows(ks, gather=gp, keep=kp)
-            v_out = gather_rows(vs, gather=gp, keep=kp)
+            k_out = gather_rows(ks, gather=gp, keep=kp, gather_checked=True)
+            v_out = gather_rows(vs, gather=gp, keep=kp, gather_checked=True)
             for i, li in enumerate(layers):
                 set_layer_kv(past_key_values, li, k_out[i], v_out[i])
         for key, layers in todo.items():
@@ -370,8 +372,10 @@ class NexusQuantEvict:
                 if kp is not None and gp is None and kept_idx is not None and key[0][2] == keep.shape[1]:
                     lst = dict(order=kept_idx, n_kept=n_kept)
                 k_out, _ = quantize_tensors(ks, is_key=True, levels=kl, rope_base=self.rope_base,
-                                            rope_scaling=self.rope_scaling, gather=gp, keep=kp, **lst)
-                v_out, _ = quantize_tensors(vs, is_key=False, levels=vl, gather=gp, keep=kp, **lst)
+                                            rope_scaling=self.rope_scaling, gather=gp, keep=kp, gather_checked=True,
+                                            **lst)
+                v_out, _ = quantize_tensors(vs, is_key=False, levels=vl, gather=gp, keep=kp, gather_checked=True,
+                                            **lst)
             for i, li in enumerate(layers):
                 set_layer_kv(past_key_values, li, k_out[i], v_out[i])
 
@@ -434,7 +438,7 @@ class NexusQuantEvictTruncate(NexusQuantEvict):
         if self.min_context_for_compression > 0 and seq < self.min_context_for_compression:
             return past_key_values, seq
         n_kept = int(n_kept_t[0].item())
-        self._apply(past_key_values, n, skip, gather=kept[0, :n_kept])
+        self._apply(past_key_values, n, skip, gather=kept[0, :n_kept], seq=seq)
         if hasattr(past_key_values, "_seen_tokens"):
             past_key_values._seen_tokens = n_kept
         return past_key_values, n_kept

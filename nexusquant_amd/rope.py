@@ -65,11 +65,15 @@ def host_table(n_pos: int, head_dim: int, base: float,
     return ang.cos(), ang.sin()
 
 
+def _scaling_key(rope_scaling: Optional[dict]) -> str:
+    return "null" if rope_scaling is None else json.dumps(rope_scaling, sort_keys=True, default=str)
+
+
 def device_table(n_pos: int, head_dim: int, base: float, rope_scaling: Optional[dict],
                  device) -> Tuple[torch.Tensor, torch.Tensor]:
     """Cached device copy of host_table covering at least n_pos positions."""
     device = torch.device(device)
-    key = (head_dim, float(base), json.dumps(rope_scaling, sort_keys=True, default=str), device)
+    key = (head_dim, float(base), _scaling_key(rope_scaling), device)
     with _lock:
         hit = _cache.get(key)
         if hit is not None and hit[0].shape[0] >= n_pos:
@@ -87,7 +91,7 @@ def device_merged_table(n_pos: int, head_dim: int, base: float, rope_scaling: Op
     host from host_table).  The fused kernels fold RoPE into the top Hadamard stage
     with these; they are the same numbers the kernels would form from cos and sin."""
     device = torch.device(device)
-    key = ("merged", head_dim, float(base), json.dumps(rope_scaling, sort_keys=True, default=str), device)
+    key = ("merged", head_dim, float(base), _scaling_key(rope_scaling), device)
     with _lock:
         hit = _cache.get(key)
         if hit is not None and hit[0].shape[0] >= n_pos:

@@ -162,6 +162,7 @@ class NexusQuantKVCompressor:
         out: List[Optional[CompressedPage]] = [None] * len(pages)
         groups: Dict[tuple, List[int]] = {}
         prepared = []
+        host_pos: Dict[torch.device, list] = {}  # positions given on the host, copied once per device
         for i, (k, v, pos) in enumerate(pages):
             _lib.require_device(k, "key_page")
             if k.dim() != 3 or v.shape != k.shape:
@@ -174,22 +175,30 @@ class NexusQuantKVCompressor:
             pos_list = torch.as_tensor(pos)
             if pos_list.numel() != n:
                 raise ValueError(f"page_positions has {pos_list.numel()} entries for {n} tokens")
+            pos_d = None
             if n and pos_list.device.type == "cpu":
-                lo, hi = int(pos_list.min()), int(pos_list.max())
+                pos_np = (pos_list.to(torch.int64) if pos_list.is_floating_point() else pos_list).numpy()
+                lo, hi = int(pos_np.min()), int(pos_np.max())
+                host_pos.setdefault(dev, []).append((i, pos_np))
             elif n:
                 lo, hi = (int(x) for x in torch.stack([pos_list.min(), pos_list.max()]).tolist())
             else:
                 lo = hi = 0
             if lo < 0:
                 raise ValueError("page positions must be non-negative")
-            pos_d = pos_list.to(device=dev, dtype=torch.int32).contiguous()
+            if not n or pos_list.device.type != "cpu":
+                pos_d = pos_list.to(device=dev, dtype=torch.int32).contiguous()
             _lib.require_device(v, "value_page")
             kk = k.contiguous()
             vv = v.contiguous()
             kk = kk if kk.data_ptr() % 16 == 0 else kk.clone()
             vv = vv if vv.data_ptr() % 16 == 0 else vv.clone()
-            prepared.append((kk, vv, pos_d, hi))
+            prepared.append([kk, vv, pos_d, hi])
             groups.setdefault((h, n, k.dtype, v.dtype, dev), []).append(i)
+        for dev, items in host_pos.items():
+            flat = torch.from_numpy(np.concatenate([p.reshape(-1).astype(np.int32) for _, p in items])).to(dev)
+            for (i, _), part in zip(items, flat.split([p.size for _, p in items])):
+                prepared[i][2] = part.reshape(torch.as_tensor(pages[i][2]).shape)
         for (h, n, kdt, vdt, dev), idx in groups.items():
             m = len(idx)
             kc = torch.empty(m, h, n, self.head_dim, dtype=torch.int8, device=dev).unbind(0)

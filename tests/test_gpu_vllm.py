@@ -370,3 +370,23 @@ def test_paged_forward_short_contexts_and_table_kinds(d, group, qdt, ctx):
     # query's type (an unrounded one alone is up to 2^-8 from a bf16 output)
     want = want.half().to(qdt)
     _close_fp16(got.float().cpu().numpy(), want.float().cpu().numpy(), bf16=qdt == torch.bfloat16)
+
+
+def test_compress_pages_takes_positions_of_any_kind():
+    """Host positions of all pages travel in one copy: lists, int64 and float tensors and
+    device tensors, mixed in one call, give the pages that single calls give."""
+    from nexusquant_amd.vllm_backend import NexusQuantKVCompressor
+    comp = NexusQuantKVCompressor(head_dim=64, bits=2)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    kinds = [list(range(5, 12)), torch.arange(7), torch.arange(100, 107, dtype=torch.int32, device=DEV),
+             torch.arange(7, dtype=torch.float32) + 30.5, torch.arange(9000, 9007, dtype=torch.int32)]
+    work = [(torch.randn(3, 7, 64, device=DEV, generator=g).half(), torch.randn(3, 7, 64, device=DEV, generator=g).half(), p)
+            for p in kinds]
+    for many, w in zip(comp.compress_pages(work), work):
+        one = comp.compress_page(*w)
+        want = torch.as_tensor(w[2]).to(torch.int32)
+        assert torch.equal(many.positions.cpu(), want.cpu()) and many.max_position == int(want.max())
+        for name in ("key_codes", "value_codes", "key_scales", "value_scales", "positions"):
+            assert torch.equal(getattr(many, name), getattr(one, name)), name
+    with pytest.raises(ValueError, match="non-negative"):
+        comp.compress_pages([(work[0][0], work[0][1], torch.arange(-1, 6))])
