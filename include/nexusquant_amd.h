@@ -31,6 +31,16 @@ extern "C" {
 #define NQ_KEEP_WRITE_KEPT 1
 #define NQ_KEEP_WRITE_EVICTED 2
 
+/*
+ * Arrays of tensor base addresses (src, recon, syms, ... of nq_quantize,
+ * nq_dequantize, nq_codes_to_int8, nq_page_encode, nq_page_decode,
+ * nq_page_logits and nq_gather_rows) are device arrays, or, with the pointer's
+ * low bit set, host arrays that are read during the call and travel in the
+ * kernel's arguments: at most NQ_MAX_HOST_ADDRESSES addresses a call in all.
+ */
+#define NQ_HOST_ARRAY(p) ((const uint64_t*)((uintptr_t)(p) | 1u))
+#define NQ_MAX_HOST_ADDRESSES 64
+
 /* element types of input tensors */
 #define NQ_F16 0
 #define NQ_BF16 1

@@ -14,6 +14,7 @@ from .build import LIB_PATH, source_hash
 
 NQ_F16, NQ_BF16, NQ_F32 = 0, 1, 2
 NQ_KEEP_ZERO, NQ_KEEP_WRITE_KEPT, NQ_KEEP_WRITE_EVICTED = 0, 1, 2
+MAX_HOST_ADDRESSES = 64  # NQ_MAX_HOST_ADDRESSES
 ABI_VERSION = 8  # NQ_ABI_VERSION of the header these bindings mirror
 _P = ctypes.c_void_p
 

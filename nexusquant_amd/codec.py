@@ -35,7 +35,7 @@ def _codes_desc(codes: Sequence[PackedCodes], outs: Sequence[torch.Tensor], rope
             raise ValueError("all codes of one launch must share shape and levels")
     dev = c0.scales.device
     staged = _PtrArrays([[c.syms for c in codes], [c.cosets for c in codes], [c.scales for c in codes],
-                         list(outs)], dev)
+                         list(outs)], dev, host=True)
     arrays = staged.arrays
     cos = sin = dm = dp = None
     n_pos = 0

@@ -23,6 +23,7 @@ struct CodecArgs {
     // dequant_kernel: 64-token tiles, (tensor, batch x head) streams, streams per block, nontemporal stores
     uint32_t n_tiles, n_sub, group, stream_out;
     float hscale;
+    InlineTabs inl;  // tables given as host arrays
 };
 
 // ---------------------------------------------------------------------------
@@ -125,7 +126,7 @@ struct RowSyms {
 template <int D, int L>
 __device__ __forceinline__ void codes_to_row(const CodecArgs& a, uint32_t tensor, size_t row, int q, uint8_t* lds_row) {
     RowSyms<D, L> rs;
-    rs.load(a.syms[tensor], a.cosets[tensor], row, q);
+    rs.load(table(a.syms)[tensor], table(a.cosets)[tensor], row, q);
     groups_to_row<D, L>(rs.d, rs.cbits, q, lds_row);
 }
 
@@ -198,6 +199,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(CodecArgs a, const uint64_
                                                       const uint64_t* __restrict__ cosets,
                                                       const uint64_t* __restrict__ scales,
                                                       const uint64_t* __restrict__ outs) {
+    const tab_t t_syms = table(syms), t_cosets = table(cosets), t_scales = table(scales), t_outs = table(outs);
     constexpr int C = D / 32;
     constexpr int RC = RopeChunks<D, DR>::value;
     // keys with DR == D: the top Hadamard stage merges with forward RoPE, as in
@@ -219,8 +221,8 @@ __global__ __launch_bounds__(256) void dequant_kernel(CodecArgs a, const uint64_
 
     float rope0[IS_KEY ? RC : 1][8], rope1[IS_KEY ? RC : 1][8];  // dm, dp or cos, sin
     RowSyms<D, L> cur;
-    cur.load(syms[tensor], cosets[tensor], (size_t)bh * a.seq + t, q);
-    float scale = gptr<const float>(scales[tensor])[(size_t)bh * a.seq + t];
+    cur.load(t_syms[tensor], t_cosets[tensor], (size_t)bh * a.seq + t, q);
+    float scale = gptr<const float>(t_scales[tensor])[(size_t)bh * a.seq + t];
     auto load_tables = [&]() {
         if constexpr (MERGED) load_rope_merged<D>(a.rope_cos, a.rope_sin, a.rope_dm, a.rope_dp, t, q, rope0, rope1);
         else if constexpr (IS_KEY) load_rope<D, DR, RC>(a.rope_cos, a.rope_sin, t, q, rope0, rope1);
@@ -249,8 +251,8 @@ __global__ __launch_bounds__(256) void dequant_kernel(CodecArgs a, const uint64_
         RowSyms<D, L> next;
         float next_scale = 0.0f;
         if constexpr (!ONE) {
-            next.load(syms[tensor], cosets[tensor], (size_t)bh * a.seq + t, q);
-            next_scale = gptr<const float>(scales[tensor])[(size_t)bh * a.seq + t];
+            next.load(t_syms[tensor], t_cosets[tensor], (size_t)bh * a.seq + t, q);
+            next_scale = gptr<const float>(t_scales[tensor])[(size_t)bh * a.seq + t];
         }
 
         half2v hp[C][4];
@@ -294,7 +296,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(CodecArgs a, const uint64_
         for (int c = 0; c < C; ++c)
 #pragma unroll
             for (int k = 0; k < 4; ++k) o[c][k] = __builtin_bit_cast(uint32_t, half2v{(__fp16)x[c][2 * k], (__fp16)x[c][2 * k + 1]});
-        store_rows16<DR>(gptr<uint8_t>(outs[tensor_c]) + ((size_t)bh_c * a.seq + t0w) * (2 * DR), min(16u, a.seq - t0w), o,
+        store_rows16<DR>(gptr<uint8_t>(t_outs[tensor_c]) + ((size_t)bh_c * a.seq + t0w) * (2 * DR), min(16u, a.seq - t0w), o,
                          stage[threadIdx.x >> 6], a.stream_out != 0);
         if constexpr (!ONE) {
             cur = next;
@@ -345,15 +347,15 @@ __global__ __launch_bounds__(256) void int8_codes_kernel(CodecArgs a) {
             }
         }
     }
-    int8_t* dst = reinterpret_cast<int8_t*>(a.out[tensor]) + row0 * D;
+    int8_t* dst = gptr<int8_t>(table(a.out)[tensor]) + row0 * D;
     // this thread's row of the next tile is loaded while the current one is
     // decoded and stored (rows past the stream read its last row, unused)
     RowSyms<D, L> next;
-    next.load(a.syms[tensor], a.cosets[tensor], row0 + min(t_begin + r, a.seq - 1u), q);
+    next.load(table(a.syms)[tensor], table(a.cosets)[tensor], row0 + min(t_begin + r, a.seq - 1u), q);
     for (uint32_t t0 = t_begin; t0 < t_end; t0 += 64) {
         const uint32_t n_rows = min(64u, t_end - t0);
         const RowSyms<D, L> cur = next;
-        if (t0 + 64 < t_end) next.load(a.syms[tensor], a.cosets[tensor], row0 + min(t0 + 64 + r, a.seq - 1u), q);
+        if (t0 + 64 < t_end) next.load(table(a.syms)[tensor], table(a.cosets)[tensor], row0 + min(t0 + 64 + r, a.seq - 1u), q);
         if (r < n_rows) groups_to_row<D, L>(cur.d, cur.cbits, q, tile + (r + 1) * STRIDE);
         __syncthreads();
         uint4 last = make_uint4(0u, 0u, 0u, 0u);
@@ -649,10 +651,12 @@ static int run_codec(const nq_codes_desc* d, int kind, void* stream) {
     const uint64_t rows = (uint64_t)d->batch * d->heads * d->seq;
     NQ_CHECK_ARG(rows < (1ull << 31), "nq codes: too many rows");
     CodecArgs a;
-    a.syms = d->syms;
-    a.cosets = d->cosets;
-    a.scales = d->scales;
-    a.out = d->out;
+    TableSet tabs{a.inl, offsetof(CodecArgs, inl)};
+    a.syms = tabs.take(d->syms, d->n_tensors);
+    a.cosets = tabs.take(d->cosets, d->n_tensors);
+    a.scales = tabs.take(d->scales, d->n_tensors);
+    a.out = tabs.take(d->out, d->n_tensors);
+    NQ_CHECK_TABLES(tabs, "nq codes");
     a.rope_cos = d->rope_cos;
     a.rope_sin = d->rope_sin;
     a.rope_dm = d->rope_sin_minus_cos;

@@ -27,6 +27,7 @@ struct PageArgs {
     uint32_t tiles;  // ceil(rows / 64)
     uint32_t rope_n_pos;
     float hscale;
+    InlineTabs inl;  // tables given as host arrays
 };
 
 // Four int8 codes (one dword) -> two fp16 pairs, exactly.  XOR 0x80 biases
@@ -41,7 +42,7 @@ __device__ __forceinline__ void codes_to_f16(uint32_t w, half2v& lo, half2v& hi)
 
 template <int D>
 __device__ __forceinline__ uint32_t page_position(const PageArgs& a, uint32_t page, uint32_t row) {
-    const int32_t p = reinterpret_cast<const int32_t*>(a.positions[page])[row % a.tokens];
+    const int32_t p = reinterpret_cast<const int32_t*>(table(a.positions)[page])[row % a.tokens];
     // the host validates positions against the table; clamp so none reads outside it
     return p < 0 ? 0u : ((uint32_t)p >= a.rope_n_pos ? a.rope_n_pos - 1u : (uint32_t)p);
 }
@@ -55,7 +56,7 @@ __global__ __launch_bounds__(256) void page_decode_kernel(PageArgs a) {
     const bool active = row_raw < a.rows;
     const uint32_t row = active ? row_raw : a.rows - 1u;  // idle quads recompute a valid row
 
-    const int8_t* crow = reinterpret_cast<const int8_t*>(a.codes[page]) + (size_t)row * D;
+    const int8_t* crow = reinterpret_cast<const int8_t*>(table(a.codes)[page]) + (size_t)row * D;
     half2v h[C][4];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(256) void page_decode_kernel(PageArgs a) {
         codes_to_f16(w.x, h[c][0], h[c][1]);
         codes_to_f16(w.y, h[c][2], h[c][3]);
     }
-    const float sc = f16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scales[page])[row]);
+    const float sc = f16_bits_to_f32(reinterpret_cast<const uint16_t*>(table(a.scales)[page])[row]);
     const float g = quad_sign(q) * ((0.5f * sc) * a.hscale);  // sign of the quad stages folded in
 
     fwht_row_f16<C, !IS_KEY>(h, q);
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(256) void page_decode_kernel(PageArgs a) {
     for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int i = 0; i < 8; ++i) asm("" : "+v"(x[c][i]));
-    uint16_t* orow = reinterpret_cast<uint16_t*>(a.out[page]) + (size_t)row * D;
+    uint16_t* orow = reinterpret_cast<uint16_t*>(table(a.out)[page]) + (size_t)row * D;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         half2v o[4];
@@ -112,7 +113,7 @@ __global__ __launch_bounds__(256) void page_logits_kernel(PageArgs a, const void
     const uint32_t row_raw = blockIdx.x * 64u + (threadIdx.x >> 2);
     const bool active = row_raw < a.rows;
     const uint32_t row = active ? row_raw : a.rows - 1u;
-    const int8_t* crow = reinterpret_cast<const int8_t*>(a.codes[0]) + (size_t)row * D;
+    const int8_t* crow = reinterpret_cast<const int8_t*>(table(a.codes)[0]) + (size_t)row * D;
     half2v h[C][4];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -120,7 +121,7 @@ __global__ __launch_bounds__(256) void page_logits_kernel(PageArgs a, const void
         codes_to_f16(w.x, h[c][0], h[c][1]);
         codes_to_f16(w.y, h[c][2], h[c][3]);
     }
-    const float sc = f16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scales[0])[row]);
+    const float sc = f16_bits_to_f32(reinterpret_cast<const uint16_t*>(table(a.scales)[0])[row]);
     const float g = quad_sign(q) * ((0.5f * sc) * a.hscale);
     fwht_row_f16<C, false>(h, q);
     float x[C][8];
@@ -221,10 +222,12 @@ extern "C" int nq_page_decode(const nq_page_desc* d, void* stream) {
     const uint64_t tiles = (rows + 63) / 64;
     NQ_CHECK_ARG(tiles * (uint64_t)d->n_pages <= max_blocks(256), "nq_page_decode: grid too large");
     PageArgs a = {};
-    a.codes = d->codes;
-    a.scales = d->scales;
-    a.positions = d->positions;
-    a.out = d->out;
+    TableSet tabs{a.inl, offsetof(PageArgs, inl)};
+    a.codes = tabs.take(d->codes, d->n_pages);
+    a.scales = tabs.take(d->scales, d->n_pages);
+    a.positions = d->is_key ? tabs.take(d->positions, d->n_pages) : nullptr;
+    a.out = tabs.take(d->out, d->n_pages);
+    NQ_CHECK_TABLES(tabs, "nq_page_decode");
     a.rope_cos = d->rope_cos;
     a.rope_sin = d->rope_sin;
     a.rope_dm = d->rope_sin_minus_cos;
@@ -266,9 +269,11 @@ extern "C" int nq_page_logits(const nq_page_desc* d, const void* query, int32_t 
     NQ_CHECK_ARG((d->rope_sin_minus_cos == nullptr) == (d->rope_cos_plus_sin == nullptr),
                  "nq_page_logits: give both or neither of rope_sin_minus_cos / rope_cos_plus_sin");
     PageArgs a = {};
-    a.codes = d->codes;
-    a.scales = d->scales;
-    a.positions = d->positions;
+    TableSet tabs{a.inl, offsetof(PageArgs, inl)};
+    a.codes = tabs.take(d->codes, 1);
+    a.scales = tabs.take(d->scales, 1);
+    a.positions = tabs.take(d->positions, 1);
+    NQ_CHECK_TABLES(tabs, "nq_page_logits");
     a.rope_cos = d->rope_cos;
     a.rope_sin = d->rope_sin;
     a.rope_dm = d->rope_sin_minus_cos;

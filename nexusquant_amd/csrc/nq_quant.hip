@@ -39,13 +39,16 @@ extern "C" int nq_quantize(const nq_quant_desc* d, void* stream) {
                      "nq_quantize: RoPE table has %lld positions, need %d",
                      (long long)d->rope_n_pos, d->seq_in > d->seq_out ? d->seq_in : d->seq_out);
     }
+    QuantArgs a;
+    memset(&a, 0, offsetof(QuantArgs, inl));
     QuantTables t = {};
-    t.src = d->src;
-    t.recon = d->recon;
-    t.syms = d->syms;
-    t.cosets = d->cosets;
-    t.scales = d->scales;
-    QuantArgs a = {};
+    TableSet tabs{a.inl, offsetof(QuantArgs, inl)};
+    t.src = tabs.take(d->src, d->n_tensors);
+    t.recon = tabs.take(d->recon, d->n_tensors);
+    t.syms = tabs.take(d->syms, d->n_tensors);
+    t.cosets = tabs.take(d->cosets, d->n_tensors);
+    t.scales = tabs.take(d->scales, d->n_tensors);
+    NQ_CHECK_TABLES(tabs, "nq_quantize");
     a.gather = d->gather;
     a.keep = d->keep;
     a.order = d->order;
@@ -123,12 +126,15 @@ extern "C" int nq_page_encode(const nq_page_desc* d, void* stream) {
         NQ_CHECK_ARG(d->rope_cos && d->rope_sin && d->rope_n_pos > 0 && d->rope_n_pos < (1ll << 31),
                      "nq_page_encode: keys need RoPE tables");
     }
+    QuantArgs a;
+    memset(&a, 0, offsetof(QuantArgs, inl));
     QuantTables t = {};
-    t.src = d->src;
-    t.positions = d->positions;
-    t.codes8 = d->codes;
-    t.scales16 = d->scales;
-    QuantArgs a = {};
+    TableSet tabs{a.inl, offsetof(QuantArgs, inl)};
+    t.src = tabs.take(d->src, d->n_pages);
+    t.positions = d->is_key ? tabs.take(d->positions, d->n_pages) : nullptr;
+    t.codes8 = tabs.take(d->codes, d->n_pages);
+    t.scales16 = tabs.take(d->scales, d->n_pages);
+    NQ_CHECK_TABLES(tabs, "nq_page_encode");
     a.rope_cos = d->rope_cos;
     a.rope_sin = d->rope_sin;
     a.rope_dm = d->rope_sin_minus_cos;

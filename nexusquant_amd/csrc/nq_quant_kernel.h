@@ -60,6 +60,7 @@ struct QuantArgs {
     const int32_t* order;
     const int32_t* n_kept;
     uint32_t stream_out;                    // the reconstructions are stored nontemporally
+    InlineTabs inl;                         // tables given as host arrays
 };
 
 // ------------------------------------------------------------------ E8 ----
@@ -712,6 +713,8 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
                                                          const uint64_t* __restrict__ tab_positions,
                                                          const uint64_t* __restrict__ tab_codes8,
                                                          const uint64_t* __restrict__ tab_scales16) {
+    const tab_t t_src = table(tab_src), t_recon = table(tab_recon), t_syms = table(tab_syms),
+                t_cosets = table(tab_cosets), t_scales = table(tab_scales);
     static_assert(!PAGE || DR == D, "page encoding takes power-of-two head dims");
     static_assert(!PAGE || SEL == kSelNone, "pages take no row selection");
     constexpr bool LIST = SEL == kSelList;
@@ -775,10 +778,10 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
             for (uint32_t j = j0; j < j1; ++j) {
                 const uint32_t tensor = j % a.n_tensors;
                 RowOut o = {};
-                o.recon = tab_recon ? gptr<uint16_t>(tab_recon[tensor]) : nullptr;
-                o.syms = tab_syms ? gptr<uint8_t>(tab_syms[tensor]) : nullptr;
-                o.cosets = tab_cosets ? gptr<uint8_t>(tab_cosets[tensor]) : nullptr;
-                o.scales = tab_scales ? gptr<float>(tab_scales[tensor]) : nullptr;
+                o.recon = tab_recon ? gptr<uint16_t>(t_recon[tensor]) : nullptr;
+                o.syms = tab_syms ? gptr<uint8_t>(t_syms[tensor]) : nullptr;
+                o.cosets = tab_cosets ? gptr<uint8_t>(t_cosets[tensor]) : nullptr;
+                o.scales = tab_scales ? gptr<float>(t_scales[tensor]) : nullptr;
                 const uint32_t bh = b * a.heads + j / a.n_tensors;
                 store_evicted_row<D, L, DR>(o, wide, bh * a.seq_out, t_out, q, in_range, a.stream_out != 0);
             }
@@ -816,7 +819,7 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
     uint8_t* wstage = stage + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * (ST::nseg * 1024);
     const uint32_t lane = threadIdx.x & 63u;
     auto stage_rows = [&](uint32_t j) {
-        const uint8_t* p = reinterpret_cast<const uint8_t*>(tab_src[j % a.n_tensors]) + row_elems(j) * ST::in_bytes;
+        const uint8_t* p = reinterpret_cast<const uint8_t*>(t_src[j % a.n_tensors]) + row_elems(j) * ST::in_bytes;
 #pragma unroll
         for (int c = 0; c < ST::chunks; ++c)
 #pragma unroll
@@ -872,7 +875,7 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
             __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
             if (j + 1 < j1) stage_rows(j + 1);
         } else {
-            const void* src = reinterpret_cast<const void*>(tab_src[tensor]);
+            const void* src = reinterpret_cast<const void*>(t_src[tensor]);
             const int64_t off = row_elems(j);
 #pragma unroll
             for (int c = 0; c < ST::chunks; ++c) load8<DT>(src, off + 32 * c, x[c]);
@@ -890,17 +893,17 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
         if constexpr (IS_KEY && PAGE) {
             // the host validates positions against the table; clamp anyway so a bad
             // position cannot read outside it
-            const int32_t pp = gptr<const int32_t>(tab_positions[tensor])[t_in % a.page_tokens];
+            const int32_t pp = gptr<const int32_t>(table(tab_positions)[tensor])[t_in % a.page_tokens];
             load_tables(pp < 0 ? 0u : ((uint32_t)pp >= a.rope_n_pos ? a.rope_n_pos - 1u : (uint32_t)pp));
         }
         RowOut o;
-        o.recon = tab_recon ? gptr<uint16_t>(tab_recon[tensor]) : nullptr;
-        o.syms = tab_syms ? gptr<uint8_t>(tab_syms[tensor]) : nullptr;
-        o.cosets = tab_cosets ? gptr<uint8_t>(tab_cosets[tensor]) : nullptr;
-        o.scales = tab_scales ? gptr<float>(tab_scales[tensor]) : nullptr;
+        o.recon = tab_recon ? gptr<uint16_t>(t_recon[tensor]) : nullptr;
+        o.syms = tab_syms ? gptr<uint8_t>(t_syms[tensor]) : nullptr;
+        o.cosets = tab_cosets ? gptr<uint8_t>(t_cosets[tensor]) : nullptr;
+        o.scales = tab_scales ? gptr<float>(t_scales[tensor]) : nullptr;
         if constexpr (PAGE) {
-            o.codes8 = gptr<int8_t>(tab_codes8[tensor]);
-            o.scales16 = tab_scales16 ? gptr<uint16_t>(tab_scales16[tensor]) : nullptr;
+            o.codes8 = gptr<int8_t>(table(tab_codes8)[tensor]);
+            o.scales16 = tab_scales16 ? gptr<uint16_t>(table(tab_scales16)[tensor]) : nullptr;
         } else {
             o.codes8 = nullptr;
             o.scales16 = nullptr;

@@ -15,6 +15,7 @@ struct RowsArgs {
     const uint8_t* keep;    // [batch, seq_in] or NULL
     uint32_t heads, seq_in, seq_out, d, chunks_per_row;  // chunks of 8 elements
     uint64_t chunks;        // total chunks per tensor
+    InlineTabs inl;         // tables given as host arrays
 };
 
 template <int DT>
@@ -38,11 +39,11 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(RowsArgs a) {
     uint4 w = make_uint4(0, 0, 0, 0);
     if (keep) {
         if constexpr (DT == NQ_F16) {
-            w = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(a.src[tensor]) + in_off);
+            w = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(table(a.src)[tensor]) + in_off);
         } else {
             float v[8];
             if constexpr (DT == NQ_BF16) {
-                uint4 r = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(a.src[tensor]) + in_off);
+                uint4 r = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(table(a.src)[tensor]) + in_off);
                 uint32_t rs[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(RowsArgs a) {
                     v[2 * k + 1] = __builtin_bit_cast(float, rs[k] & 0xffff0000u);
                 }
             } else {
-                const float4* p = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(a.src[tensor]) + in_off);
+                const float4* p = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(table(a.src)[tensor]) + in_off);
                 float4 x0 = p[0], x1 = p[1];
                 v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w;
                 v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(RowsArgs a) {
             w.w = f32_to_f16_bits(v[6]) | (f32_to_f16_bits(v[7]) << 16);
         }
     }
-    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.dst[tensor]) + out_off) = w;
+    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(table(a.dst)[tensor]) + out_off) = w;
 }
 
 }  // namespace nq
@@ -78,8 +79,10 @@ extern "C" int nq_gather_rows(const uint64_t* src, const uint64_t* dst, int32_t 
     NQ_CHECK_ARG(gather || seq_in == seq_out, "nq_gather_rows: seq_out must equal seq_in without gather");
     if (n_tensors == 0 || seq_out == 0) return NQ_OK;
     RowsArgs a;
-    a.src = src;
-    a.dst = dst;
+    TableSet tabs{a.inl, offsetof(RowsArgs, inl)};
+    a.src = tabs.take(src, n_tensors);
+    a.dst = tabs.take(dst, n_tensors);
+    NQ_CHECK_TABLES(tabs, "nq_gather_rows");
     a.gather = gather;
     a.keep = keep;
     a.heads = (uint32_t)heads;

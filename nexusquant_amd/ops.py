@@ -128,10 +128,12 @@ def _ring(device) -> _AddressRing:
 
 class _PtrArrays:
     """Device addresses of int64 arrays of the base addresses of each tensor
-    group, staged through the device's address ring.  Call release() right after
-    the launch that reads them."""
+    group, staged through the device's address ring; with host=True and at most
+    NQ_MAX_HOST_ADDRESSES addresses, tagged addresses of host arrays instead, for
+    the entry points that take those into the launch's arguments.  Call release()
+    right after the launch that reads them (and keep the object until then)."""
 
-    def __init__(self, groups: Sequence[Optional[Sequence[torch.Tensor]]], device):
+    def __init__(self, groups: Sequence[Optional[Sequence[torch.Tensor]]], device, host: bool = False):
         flat: List[int] = []
         spans = []
         for g in groups:
@@ -145,8 +147,12 @@ class _PtrArrays:
         if not flat:
             self.arrays = [None for _ in groups]
             return
-        self._ring = _ring(device)
-        dev, self._span = self._ring.stage(flat)
+        if host and len(flat) <= _lib.MAX_HOST_ADDRESSES:
+            self._host = (ctypes.c_uint64 * len(flat))(*flat)
+            dev = ctypes.addressof(self._host) | 1
+        else:
+            self._ring = _ring(device)
+            dev, self._span = self._ring.stage(flat)
         self.arrays = [None if sp is None else dev + 8 * sp[0] for sp in spans]
 
     def release(self) -> None:
@@ -310,7 +316,7 @@ def quantize_tensors(tensors: Sequence[torch.Tensor], *, is_key: bool, levels: i
               [c.syms for c in codes_t] if codes_t else None,
               [c.cosets for c in codes_t] if codes_t else None,
               [c.scales for c in codes_t] if codes_t else None]
-    staged = _PtrArrays(groups, dev)
+    staged = _PtrArrays(groups, dev, host=True)
     arrays = dict(zip(names, staged.arrays))
     desc = _lib.QuantDesc(
         n_tensors=n, batch=b, heads=h, seq_in=s, seq_out=seq_out, head_dim=d,
@@ -511,7 +517,7 @@ def gather_rows(tensors: Sequence[torch.Tensor], *, gather: Optional[torch.Tenso
         if tuple(k.shape) != (b, s):
             raise ValueError(f"keep must be [batch, seq] = {(b, s)}")
     out = list(torch.empty(len(src), b, h, seq_out, d, dtype=torch.float16, device=dev).unbind(0))
-    staged = _PtrArrays([src, out], dev)
+    staged = _PtrArrays([src, out], dev, host=True)
     arr_src, arr_dst = staged.arrays
     with torch.cuda.device(dev):
         try:

@@ -212,7 +212,7 @@ class NexusQuantKVCompressor:
                 codes = kc if is_key else vc
                 scales = ks if is_key else vs
                 groups_t = [src, [prepared[i][2] for i in idx] if is_key else None, list(codes), list(scales)]
-                staged = _PtrArrays(groups_t, dev)
+                staged = _PtrArrays(groups_t, dev, host=True)
                 arrays = dict(zip(("src", "positions", "codes", "scales"), staged.arrays))
                 desc = self._desc(m, h, n, is_key, arrays, tables, _lib.dtype_code(kdt if is_key else vdt))
                 with torch.cuda.device(dev):
@@ -250,7 +250,7 @@ class NexusQuantKVCompressor:
                                 [p.key_scales if is_key else p.value_scales for p in pg],
                                 [p.positions for p in pg] if is_key else None,
                                 list(ko if is_key else vo)]
-                    staged = _PtrArrays(groups_t, dev)
+                    staged = _PtrArrays(groups_t, dev, host=True)
                     arrays = dict(zip(("codes", "scales", "positions", "out"), staged.arrays))
                     desc = self._desc(m, h, n, is_key, arrays, tables)
                     with torch.cuda.device(dev):
@@ -281,7 +281,7 @@ class NexusQuantKVCompressor:
         if n == 0 or q_len == 0:
             return logits
         tables = self._tables(_page_max_position(p), dev)
-        staged = _PtrArrays([[p.key_codes], [p.key_scales], [p.positions]], dev)
+        staged = _PtrArrays([[p.key_codes], [p.key_scales], [p.positions]], dev, host=True)
         arrays = dict(zip(("codes", "scales", "positions"), staged.arrays))
         desc = self._desc(1, h, n, True, arrays, tables)
         with torch.cuda.device(dev):
