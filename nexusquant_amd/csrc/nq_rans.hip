@@ -37,17 +37,22 @@ __device__ __forceinline__ int hist_bin(int8_t c, int L) {
 // hs = 65 (the earlier layout) copy c + 1's bin b - 1 shared copy c's bin b's
 // bank, and one instruction's busiest bank held about 7 lanes instead of 4.
 // Levels 16 (33 bins) keep hs = 65.  (One copy per lane measured the same.)
+// Two blocks of 1024 threads per CU: every block adds its bins to the same few
+// global words, and with 4096 blocks of 256 those 70000 atomics were most of a
+// layer's histogram (33.5 M codes at 17 bins, kernel trace: 51.4 -> 13.4 us).
 constexpr int kHistCopies = 16;
 constexpr int kHistStride = kRansMaxAlpha + 1;
+constexpr int kHistThreads = 1024;
+constexpr int64_t kHistBlocks = 512;
 
-__global__ __launch_bounds__(256) void rans_hist_kernel(const int8_t* codes, int64_t n, int L, uint32_t* hist) {
+__global__ __launch_bounds__(kHistThreads) void rans_hist_kernel(const int8_t* codes, int64_t n, int L, uint32_t* hist) {
     __shared__ uint32_t h_all[kHistCopies * kHistStride];
-    for (int i = threadIdx.x; i < kHistCopies * kHistStride; i += 256) h_all[i] = 0;
+    for (int i = threadIdx.x; i < kHistCopies * kHistStride; i += kHistThreads) h_all[i] = 0;
     __syncthreads();
     const int hs = 2 * L + 1 <= 17 ? 17 : kHistStride;  // words between copies
     uint32_t* const h = h_all + (threadIdx.x & (kHistCopies - 1)) * hs;
-    const int64_t stride = (int64_t)gridDim.x * 256 * 16;
-    for (int64_t base = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 16; base < n; base += stride) {
+    const int64_t stride = (int64_t)gridDim.x * kHistThreads * 16;
+    for (int64_t base = ((int64_t)blockIdx.x * kHistThreads + threadIdx.x) * 16; base < n; base += stride) {
         if (base + 16 <= n) {
             const uint4 w = *reinterpret_cast<const uint4*>(codes + base);
             const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
@@ -78,7 +83,7 @@ constexpr int kHistSmallBins = 9;
 constexpr int kHistSmallLoads = 4;  // 16-byte loads per lane in flight: 64 codes between flushes
                                     // (8 in flight, flushed every 4, measured the same)
 
-__global__ __launch_bounds__(256) void rans_hist_small_kernel(const int8_t* codes, int64_t n, int L, uint32_t* hist) {
+__global__ __launch_bounds__(kHistThreads) void rans_hist_small_kernel(const int8_t* codes, int64_t n, int L, uint32_t* hist) {
     __shared__ uint32_t h[kHistSmallBins];
     if (threadIdx.x < kHistSmallBins) h[threadIdx.x] = 0;
     __syncthreads();
@@ -103,8 +108,8 @@ __global__ __launch_bounds__(256) void rans_hist_small_kernel(const int8_t* code
     };
     const uint4* const v = reinterpret_cast<const uint4*>(codes);
     const int64_t n16 = n / 16;
-    const int64_t stride = (int64_t)gridDim.x * 256;
-    int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * kHistThreads;
+    int64_t g = (int64_t)blockIdx.x * kHistThreads + threadIdx.x;
     for (; g + (kHistSmallLoads - 1) * stride < n16; g += kHistSmallLoads * stride) {
         uint4 w[kHistSmallLoads];
 #pragma unroll
@@ -761,13 +766,12 @@ extern "C" int nq_rans_histogram(const int8_t* codes, int64_t n, int32_t levels,
                  (long long)n);
     NQ_CHECK_ARG(((uintptr_t)codes & 15) == 0, "nq_rans_histogram: codes must be 16-byte aligned");
     if (n == 0) return NQ_OK;
-    int64_t blocks = (n + 256 * 16 - 1) / (256 * 16);
-    if (blocks > 4096) blocks = 4096;
+    const int64_t blocks = std::min<int64_t>((n + kHistThreads * 16 - 1) / (kHistThreads * 16), kHistBlocks);
     if (2 * levels + 1 <= kHistSmallBins)
-        hipLaunchKernelGGL(rans_hist_small_kernel, dim3((uint32_t)blocks), dim3(256), 0, (hipStream_t)stream, codes, n,
+        hipLaunchKernelGGL(rans_hist_small_kernel, dim3((uint32_t)blocks), dim3(kHistThreads), 0, (hipStream_t)stream, codes, n,
                            levels, hist);
     else
-        hipLaunchKernelGGL(rans_hist_kernel, dim3((uint32_t)blocks), dim3(256), 0, (hipStream_t)stream, codes, n,
+        hipLaunchKernelGGL(rans_hist_kernel, dim3((uint32_t)blocks), dim3(kHistThreads), 0, (hipStream_t)stream, codes, n,
                            levels, hist);
     NQ_CHECK_HIP(hipGetLastError());
     return NQ_OK;

@@ -196,3 +196,15 @@ def test_encode_many_and_decode_many_equal_the_single_calls():
     back = rans_decode_many(many)
     for t, b in zip(tensors, back):
         assert torch.equal(b, t)
+
+
+@pytest.mark.parametrize("levels", [2, 4, 8, 16])
+@pytest.mark.parametrize("n", [1, 15, 16, 16383, 16384, 16385, 512 * 16384 - 1, 512 * 16384 + 17, 3 * 512 * 16384 + 5])
+def test_histogram_at_the_grid_edges(levels, n):
+    """One block's run of codes (16384), the whole grid's, and the steps after them."""
+    from nexusquant_amd.entropy import _code_counts
+    print(f"[gpu] histogram n={n} levels={levels}", flush=True)
+    g = torch.Generator(device="cuda:0").manual_seed(n + levels)
+    c = (torch.randn(n, device="cuda:0", generator=g) * levels / 3).round().clamp(-levels, levels).to(torch.int8)
+    want = torch.bincount((c.to(torch.int32) + levels), minlength=2 * levels + 1).cpu().numpy()
+    assert np.array_equal(_code_counts(c, levels), want)
