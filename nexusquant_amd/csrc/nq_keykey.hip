@@ -63,6 +63,7 @@ struct Args {
     float2* part;       // [bh, nsplit, nq] (m, z) per split and query
     float* importance;  // [batch, seq]
     int32_t seq, obs, nq, nsplit, split_keys, heads, batch;
+    int32_t combined;   // kk_combine has put each query's final (m, z) at split 0
     float scale;
 };
 
@@ -232,6 +233,30 @@ __global__ __launch_bounds__(256) void kk_stats(Args a) {
     }
 }
 
+// One wave per (batch, head, query block): the splits' partials of 32 queries
+// into split 0's slot, in the order kk_colsum itself combines them (alternate
+// splits in lanes c and c + 32), so the result is the same to the bit.  Without it
+// every workgroup of kk_colsum runs the whole chain, nsplit / 2 dependent steps.
+__global__ __launch_bounds__(64) void kk_combine(Args a) {
+    const int lane = threadIdx.x, g = lane >> 5, c = lane & 31;
+    const int n_qb = a.nq / kQueryBlock;
+    const int bh = blockIdx.x / n_qb, qb = blockIdx.x % n_qb;
+    float2* part = a.part + (size_t)bh * a.nsplit * a.nq + qb * kQueryBlock + c;
+    float2 s = make_float2(-__builtin_inff(), 0.0f);
+    constexpr int U = 8;  // loads in flight
+    int sp = g;
+    for (; sp + 2 * (U - 1) < a.nsplit; sp += 2 * U) {
+        float2 v[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) v[k] = part[(size_t)(sp + 2 * k) * a.nq];
+#pragma unroll
+        for (int k = 0; k < U; ++k) s = combine(s, v[k]);
+    }
+    for (; sp < a.nsplit; sp += 2) s = combine(s, part[(size_t)sp * a.nq]);
+    s = combine(s, make_float2(__shfl_xor(s.x, 32, 64), __shfl_xor(s.y, 32, 64)));
+    if (g == 0) part[0] = s;  // read by this lane alone, above
+}
+
 // grid: batch * ceil(seq / (32 KT)) workgroups of W = min(heads, 8) waves;
 // wave w takes heads w, w + W, ... of KT 32-key tiles of one batch row.
 template <int DT, int D, int KT>
@@ -264,8 +289,12 @@ __global__ __launch_bounds__(64 * kMaxWaves) void kk_colsum(Args a) {
             // row maximum and sum of query 32 qb + c: the splits' partials,
             // alternate splits in lanes c and c + 32 (fixed order: deterministic)
             float2 s = make_float2(-__builtin_inff(), 0.0f);
-            for (int sp = g; sp < a.nsplit; sp += 2) s = combine(s, part[(size_t)sp * a.nq + qb * kQueryBlock + c]);
-            s = combine(s, make_float2(__shfl_xor(s.x, 32, 64), __shfl_xor(s.y, 32, 64)));
+            if (a.combined) {
+                s = part[qb * kQueryBlock + c];
+            } else {
+                for (int sp = g; sp < a.nsplit; sp += 2) s = combine(s, part[(size_t)sp * a.nq + qb * kQueryBlock + c]);
+                s = combine(s, make_float2(__shfl_xor(s.x, 32, 64), __shfl_xor(s.y, 32, 64)));
+            }
             // LDS ops of one wave execute in order; the fences keep the compiler
             // from moving the reads below above the write.  Rows past obs get
             // M = +inf and 1/Z = 0, so their terms are exp2(-inf) * 0 = 0.
@@ -321,7 +350,16 @@ __global__ __launch_bounds__(64 * kMaxWaves) void kk_colsum(Args a) {
 }
 
 constexpr int kTilesPerWave = 4;  // kk_stats: 32-key tiles per wave
-constexpr int kColsumTiles = 4;   // kk_colsum: 32-key tiles per wave
+// kk_colsum: 32-key tiles per wave (KT): 4, which reads a head's queries once per
+// 128 keys, when that leaves a workgroup for each CU, else 2 or 1.  Scores of one
+// batch row, call between events, us (4 always -> this rule): 8 heads x 500 keys
+// 21.8 -> 16.7, x 8191 25.3 -> 20.2, 32 heads x 8192 66 -> 46; four rows of 8 heads
+// x 8192 stay at 4 (33; 38 at 2).
+constexpr int kColsumTiles = 4;
+constexpr int64_t kColsumBlocks = 256;
+// Splits (of 512 keys) from which kk_combine's launch costs less than the chains
+// it replaces: 8 heads x 65521 keys 105 -> 66 us, x 131072 287 -> 122.
+constexpr int kCombineSplits = 32;
 constexpr int kSplitKeys = 4 * 32 * kTilesPerWave;
 
 int64_t workspace_bytes(int64_t bh, int64_t seq, int64_t nq) {
@@ -333,9 +371,16 @@ template <int DT, int D>
 hipError_t launch(const Args& a, hipStream_t st) {
     const int bh = a.batch * a.heads;
     hipLaunchKernelGGL((kk_stats<DT, D, kTilesPerWave>), dim3(bh * a.nsplit), dim3(256), 0, st, a);
-    const int n_kr = (a.seq + 32 * kColsumTiles - 1) / (32 * kColsumTiles);
+    Args c = a;
+    c.combined = a.nsplit >= kCombineSplits;
+    if (c.combined) hipLaunchKernelGGL(kk_combine, dim3(bh * (a.nq / kQueryBlock)), dim3(64), 0, st, c);
     const int waves = a.heads < kMaxWaves ? a.heads : kMaxWaves;
-    hipLaunchKernelGGL((kk_colsum<DT, D, kColsumTiles>), dim3(a.batch * n_kr), dim3(64 * waves), 0, st, a);
+    int kt = kColsumTiles;
+    while (kt > 1 && (int64_t)a.batch * ((a.seq + 32 * kt - 1) / (32 * kt)) < kColsumBlocks) kt >>= 1;
+    const dim3 grid(a.batch * ((a.seq + 32 * kt - 1) / (32 * kt))), block(64 * waves);
+    if (kt == 4) hipLaunchKernelGGL((kk_colsum<DT, D, 4>), grid, block, 0, st, c);
+    else if (kt == 2) hipLaunchKernelGGL((kk_colsum<DT, D, 2>), grid, block, 0, st, c);
+    else hipLaunchKernelGGL((kk_colsum<DT, D, 1>), grid, block, 0, st, c);
     return hipGetLastError();
 }
 
@@ -380,6 +425,7 @@ int score_keykey_ws(const void* keys, int32_t dtype, int32_t batch, int32_t head
     a.heads = heads;
     a.batch = batch;
     a.scale = scale;
+    a.combined = 0;
     a.part = static_cast<float2*>(workspace);
     a.importance = importance;
     hipStream_t st = (hipStream_t)stream;
