@@ -198,8 +198,8 @@ int nq_score_real(const void* q, const void* k, int32_t dtype, int32_t batch, in
  * in fp32 on the matrix cores.  fp16 / bf16, head_dim 64 or 128, 16-byte aligned
  * tensors; v [batch, kv_heads, seq, head_dim]; sliding_window and logit_map as
  * for nq_score_real.  workspace:
- * nq_attention_real_workspace bytes (row statistics, column sums and V
- * transposed with the keys of each 32-key block in the accumulator's order).
+ * nq_attention_real_workspace bytes (nq_score_real's and V transposed with the
+ * keys of each 32-key block in the accumulator's order).
  *
  * Replaces: eager_attention_forward (transformers modeling_llama.py:179-213) in
  *           the scoring forward of _score_importance_real  pipeline.py:784-836

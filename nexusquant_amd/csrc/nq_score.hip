@@ -3,6 +3,8 @@
 // The key-key scorer is in nq_keykey.hip.
 #include "nq_common.h"
 
+#include <algorithm>
+
 namespace nq {
 
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -202,10 +204,10 @@ __global__ __launch_bounds__(64) void real_sweep(RealArgs a) {
 // alone) and the sum z of exp(x - max) relative to it, rescaling z when m
 // grows; lanes c and c + 32 (the same query) are combined at the end.  Writes
 // -max * log2(e) and 1 / sum per row.
-// real_colsum: a workgroup owns 128 keys (wave w: keys 32w..32w+31) as the B
-// operand and streams the query tiles from its first key on; it accumulates
-// round_T(exp(x - max) / sum) per key column in registers (fixed order, so the
-// result does not depend on scheduling) and writes the column sums.
+// real_output: the same work items with the rows' final statistics; it forms
+// round_T(exp(x - max) / sum), sums it per key (tile_sums, in a fixed order, so
+// the result does not depend on scheduling) and, for the attention output, feeds
+// it to P V.
 // exp is v_exp_f32 on x * log2(e) - max * log2(e) and the division a multiply
 // by the row's reciprocal sum: within a few ulp of the eager fp32 softmax.
 // ---------------------------------------------------------------------------
@@ -235,31 +237,6 @@ __device__ __forceinline__ f32x16 mfma16(uint4 a, uint4 b, f32x16 acc) {
                                                        acc, 0, 0, 0);
 }
 
-// 16-byte units of rows [row0, row0 + 64) of a [seq, D] matrix (rows clamped to seq - 1).
-// Every thread loads PER_THREAD units unconditionally (UNITS is a multiple of
-// 256 for every supported D), so the loads issue back to back and only the
-// LDS store waits for them.
-template <int D>
-__device__ __forceinline__ void tile_load(const uint16_t* base, int row0, int seq, uint4 (&r)[RealTile<D>::PER_THREAD]) {
-    static_assert(RealTile<D>::UNITS % 256 == 0, "64-row stages of 16-byte units fill 256 threads evenly");
-#pragma unroll
-    for (int k = 0; k < RealTile<D>::PER_THREAD; ++k) {
-        const int u = threadIdx.x + 256 * k;
-        int row = row0 + u / (D / 8);
-        row = row < seq ? row : seq - 1;
-        r[k] = *reinterpret_cast<const uint4*>(base + (size_t)row * D + (u % (D / 8)) * 8);
-    }
-}
-
-template <int D>
-__device__ __forceinline__ void tile_store(char* lds, const uint4 (&r)[RealTile<D>::PER_THREAD]) {
-#pragma unroll
-    for (int k = 0; k < RealTile<D>::PER_THREAD; ++k) {
-        const int u = threadIdx.x + 256 * k;
-        *reinterpret_cast<uint4*>(lds + (u / (D / 8)) * RealTile<D>::ROWB + (u % (D / 8)) * 16) = r[k];
-    }
-}
-
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) void global_void_t;
 
@@ -267,7 +244,7 @@ typedef __attribute__((address_space(1))) void global_void_t;
 constexpr int kWaitVm0 = 0x0f70;
 
 // Rows [row0, row0 + 64) of a [seq, D] matrix into one LDS stage by direct-to-LDS
-// loads, in the padded layout tile_store writes (row r at r * ROWB).  The stage
+// loads, row r at byte r * ROWB.  The stage
 // is UPR = ROWB / 16 windows of 64 16-byte slots; window w goes to wave w mod 4,
 // and lane l of it fills slot 64 w + l: row (64 w + l) / UPR, unit
 // (64 w + l) mod UPR, the pad unit (D / 8) masked off.  Nothing passes through
@@ -326,17 +303,6 @@ __device__ __forceinline__ void tile_dma(const DmaPlan<D>& plan, const uint16_t*
             }
         }
     }
-}
-
-// 32x32 logits: A from registers (this lane's row, K chunks), B from 32 LDS rows.
-template <int DT, int D>
-__device__ __forceinline__ f32x16 logits_regs_lds(const uint4 (&a)[RealTile<D>::KS], const char* lds, int c, int g) {
-    f32x16 acc = {};
-    const char* row = lds + c * RealTile<D>::ROWB + 16 * g;
-#pragma unroll
-    for (int s = 0; s < RealTile<D>::KS; ++s)
-        acc = mfma16<DT>(a[s], *reinterpret_cast<const uint4*>(row + 32 * s), acc);
-    return acc;
 }
 
 // 32x32 logits: A (queries) from 32 LDS rows, B (keys) from registers.
@@ -601,154 +567,28 @@ __device__ __forceinline__ f32x4 mfma16x16(uint4 a, uint4 b, f32x4 acc) {
                                                        acc, 0, 0, 0);
 }
 
-// Column sums of one 32 x 32 tile of a lane's key column (queries = rows
-// acc_row(j, g)): p = round_T(exp2(x * log2(e) + nm[row]) * rz[row]) with x the
-// eager logit, then colacc += P^T . B on the matrix cores with two 16x16x32
-// MFMAs (8 rounded values per lane each).  As their A operand, lane l's 8
-// values are row l % 16, K slice l / 16; that lane holds key l % 32 = row +
-// 16 ((l / 16) & 1).  B (ones_sel) is 1 where column 0 meets the slices of key
-// row and column 1 those of key row + 16, else 0, so column 0 of the result
-// accumulates the sums of keys 0..15 and column 1 those of keys 16..31, in
-// fp32.  That is half the matrix-core passes of summing against an all-ones
-// 32x32x16 operand.  MASKED: rows r with r < key_off (row before the key) or
-// r >= row_end (past seq, or at or past key + window) contribute 0.
-template <int DT, bool MASKED, bool MAP = false>
-__device__ __forceinline__ void col_fold(const f32x16& acc, const float* nm_rows, const float* rz_rows, float scaling,
-                                         int key_off, int row_end, int g, const uint4& ones_sel, f32x4& colacc,
-                                         const uint16_t* map = nullptr) {
-    uint32_t pk[8];
-#pragma unroll
-    for (int jq = 0; jq < 4; ++jq) {
-        const int r0 = 8 * jq + 4 * g;  // rows r0 .. r0 + 3 of the 32-row block
-        const float4 nm4 = *reinterpret_cast<const float4*>(&nm_rows[r0]);
-        const float4 rz4 = *reinterpret_cast<const float4*>(&rz_rows[r0]);
-        const float nm[4] = {nm4.x, nm4.y, nm4.z, nm4.w};
-        const float rz[4] = {rz4.x, rz4.y, rz4.z, rz4.w};
-#pragma unroll
-        for (int u = 0; u < 4; u += 2) {
-            const int j = 4 * jq + u;
-            float x0, x1;
-            exp_args2<DT, MAP>(acc[j], acc[j + 1], scaling, nm[u], nm[u + 1], x0, x1, map);
-            float p0 = __builtin_amdgcn_exp2f(x0) * rz[u];
-            float p1 = __builtin_amdgcn_exp2f(x1) * rz[u + 1];
-            if constexpr (MASKED) {
-                const int r = r0 + u;
-                p0 = key_off <= r && r < row_end ? p0 : 0.0f;
-                p1 = key_off <= r + 1 && r + 1 < row_end ? p1 : 0.0f;
-            }
-            pk[j / 2] = round_pair<DT>(p0, p1);
-        }
-    }
-    colacc = mfma16x16<DT>(make_uint4(pk[0], pk[1], pk[2], pk[3]), ones_sel, colacc);
-    colacc = mfma16x16<DT>(make_uint4(pk[4], pk[5], pk[6], pk[7]), ones_sel, colacc);
+// Column sums of one 32 x 32 tile of probabilities, pk packed so that lane l
+// holds key l % 32 at the 16 queries acc_row(., l / 32), on the matrix cores
+// with two 16x16x32 MFMAs.  As their A operand, lane l's 8 values are row
+// l % 16, K slice l / 16; that lane holds key l % 32 = row + 16 ((l / 16) & 1).
+// B (ones_select) is 1 where column 0 meets the slices of key row and column 1
+// those of key row + 16, else 0, so lane l with l % 16 = n < 2 gets the sums of
+// keys 4 (l / 16) + i + 16 n.  That is half the matrix-core passes of summing
+// against an all-ones 32x32x16 operand.
+// The four tiles of a 128-query block are added up first, then the blocks
+// (block_sums), in that order at every size.
+template <int DT>
+__device__ __forceinline__ f32x4 tile_sums(const uint32_t (&pk)[8], const uint4& ones_sel) {
+    f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+    t = mfma16x16<DT>(make_uint4(pk[0], pk[1], pk[2], pk[3]), ones_sel, t);
+    return mfma16x16<DT>(make_uint4(pk[4], pk[5], pk[6], pk[7]), ones_sel, t);
 }
 
-template <int DT, int D, bool MAP = false, bool WIN = false>
-__global__ __launch_bounds__(256) void real_colsum(RealArgs a) {
-    __shared__ __align__(16) char lds0[RealTile<D>::BUF];
-    __shared__ __align__(16) char lds1[RealTile<D>::BUF];
-    __shared__ __align__(16) float st_nm0[64], st_rz0[64], st_nm1[64], st_rz1[64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 5, c = lane & 31;
-    // items ordered (batch x query head, key block): an XCD range walks its
-    // query heads one after the other, so the streamed queries stay in its L2
-    const int item = xcd_item(a);
-    if (item >= a.n_items) return;
-    const int n_blocks = (a.seq + 127) / 128;
-    const int kb = item % n_blocks;                  // first key blocks see the most queries
-    const int bhq = item / n_blocks;
-    const int b = bhq / a.hq, hq = bhq - b * a.hq;
-    const int hk = hq / (a.hq / a.hkv);
-    const uint16_t* qbase = static_cast<const uint16_t*>(a.q) + (size_t)bhq * a.seq * D;
-    const uint16_t* kbase = static_cast<const uint16_t*>(a.k) + ((size_t)b * a.hkv + hk) * a.seq * D;
-    const size_t stat = (size_t)bhq * a.seq;
-    const int k0 = kb * 128 + wave * 32;            // this wave's first key
-    const int key = k0 + c;
-    const int my_first = k0 / 32;                    // first 32-row query block that sees these keys
-    const int it0 = kb * 2;                          // first 64-row query stage of the block
-    const int W = WIN ? a.window : kNoWindow;
-    // one past the last 64-row stage holding a query that sees a key of the block
-    // (key j is seen by queries j .. j + W - 1)
-    const int n_it = WIN ? min((a.seq + 63) / 64, (kb * 128 + 126 + W) / 64 + 1) : (a.seq + 63) / 64;
-    const bool live = k0 < a.seq;
-    // a query tile is whole for this wave's keys [k0, k0 + 31] when all its rows
-    // come after them, lie below seq and (WIN) before k0 + W; none when all its
-    // rows come before the keys or (WIN) at or past k0 + 31 + W
-    auto q_whole = [&](int qt) {
-        return qt > my_first && qt * 32 + 32 <= a.seq && (!WIN || qt * 32 + 31 < k0 + W);
-    };
-    auto q_none = [&](int qt) { return qt < my_first || (WIN && qt * 32 >= k0 + 31 + W); };
-    uint4 kr[RealTile<D>::KS];
-    row_operand<D>(kbase, key, a.seq, g, kr);
-    f32x4 colacc = {0.0f, 0.0f, 0.0f, 0.0f};
-    // 16x16x32 B operand: column n of lane l is l % 16, its K slice l / 16; a
-    // slice holds key (l % 32) = row + 16 ((l / 16) & 1), so column 0 sums the
-    // slices of key row and column 1 those of key row + 16
-    uint4 ones_sel;
-    {
-        constexpr uint32_t one2 = DT == NQ_F16 ? 0x3C003C00u : 0x3F803F80u;
-        const uint32_t v = (lane & 15) == ((lane >> 4) & 1) ? one2 : 0u;
-        ones_sel = make_uint4(v, v, v, v);
-    }
-    // One stage: 64 query rows by direct-to-LDS loads, and (wave 0) their row
-    // statistics, one dword per lane.  Two buffers in fixed roles as in
-    // real_rowstats; each thread waits for its own loads before the barrier.
-    const DmaPlan<D> plan;
-    auto load_stage = [&](int it, char* buf, float* nm, float* rz) {
-        tile_dma<D>(plan, qbase, it * 64, a.seq, buf);
-        if (wave == 0) {
-            const int i = min(it * 64 + lane, a.seq - 1);
-            __builtin_amdgcn_global_load_lds((global_void_t*)(a.row_max + stat + i), (lds_void_t*)nm, 4, 0, 0);
-            __builtin_amdgcn_global_load_lds((global_void_t*)(a.row_sum + stat + i), (lds_void_t*)rz, 4, 0, 0);
-        }
-    };
-    load_stage(it0, lds0, st_nm0, st_rz0);
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
-    __syncthreads();
-    auto stage = [&](int it, const char* cur, const float* cnm, const float* crz, char* nxt, float* nnm,
-                     float* nrz) {
-        if (it + 1 < n_it) load_stage(it + 1, nxt, nnm, nrz);
-        if (live) {
-            const int qt0 = 2 * it;
-            if (qt0 > my_first && qt0 * 32 + 64 <= a.seq && (!WIN || qt0 * 32 + 63 < k0 + W)) {
-                // both blocks interior: one basic block, so the second tile's
-                // MFMAs run under the first tile's VALU work
-                const f32x16 acc0 = logits_lds_regs<DT, D>(cur, kr, c, g);
-                const f32x16 acc1 = logits_lds_regs<DT, D>(cur + 32 * RealTile<D>::ROWB, kr, c, g);
-                col_fold<DT, false, MAP>(acc0, cnm, crz, a.scaling, 0, 0, g, ones_sel, colacc, a.logit_map);
-                col_fold<DT, false, MAP>(acc1, cnm + 32, crz + 32, a.scaling, 0, 0, g, ones_sel, colacc,
-                                         a.logit_map);
-            } else {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int qt = qt0 + h;
-                    if (q_none(qt)) continue;
-                    const f32x16 acc = logits_lds_regs<DT, D>(cur + h * 32 * RealTile<D>::ROWB, kr, c, g);
-                    if (q_whole(qt))
-                        col_fold<DT, false, MAP>(acc, cnm + 32 * h, crz + 32 * h, a.scaling, 0, 0, g, ones_sel,
-                                                 colacc, a.logit_map);
-                    else
-                        col_fold<DT, true, MAP>(acc, cnm + 32 * h, crz + 32 * h, a.scaling, key - qt * 32,
-                                                WIN ? min(a.seq, key + W) - qt * 32 : a.seq - qt * 32, g, ones_sel,
-                                                colacc, a.logit_map);
-                }
-            }
-        }
-        __builtin_amdgcn_s_waitcnt(kWaitVm0);  // this thread's part of the next stage has landed
-        __syncthreads();
-    };
-#pragma unroll 1
-    for (int it = it0; it < n_it; it += 2) {
-        stage(it, lds0, st_nm0, st_rz0, lds1, st_nm1, st_rz1);
-        if (it + 1 < n_it) stage(it + 1, lds1, st_nm1, st_rz1, lds0, st_nm0, st_rz0);
-    }
-    // lane l (column n = l % 16 < 2) holds the sums of keys k0 + 4 (l / 16) + i + 16 n
-    if ((lane & 15) < 2 && live) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int kk = k0 + 4 * (lane >> 4) + i + 16 * (lane & 15);
-            if (kk < a.seq) a.colsum[stat + kk] = colacc[i];
-        }
-    }
+template <int DT>
+__device__ __forceinline__ uint4 ones_select(int lane) {
+    constexpr uint32_t one2 = DT == NQ_F16 ? 0x3C003C00u : 0x3F803F80u;
+    const uint32_t v = (lane & 15) == ((lane >> 4) & 1) ? one2 : 0u;
+    return make_uint4(v, v, v, v);
 }
 
 // ---------------------------------------------------------------------------
@@ -849,7 +689,9 @@ struct OutArgs {
     RealArgs r;
     const uint16_t* vt;  // [batch * hkv, D, s64]
     void* out;           // [batch, hq, seq, D] in the model dtype
+    float* partial;      // COL: [batch * hq, qb_n, s64] column sums of one 128-query block each
     int32_t s64;
+    int32_t qb0, qb_n;   // the launch's query blocks [qb0, qb0 + qb_n)
 };
 
 // Rounded probabilities of one 32 x 32 logit tile for this lane's query (nm,
@@ -890,31 +732,72 @@ __device__ __forceinline__ void out_pv(const uint4 (&pa)[2], const char* vbuf, i
     }
 }
 
+// tile_sums of the 32 x 32 tile of rounded probabilities that feeds P V.  There a
+// lane holds a query's keys, so the tile is first transposed on the matrix cores:
+// P times the slot-order permutation (sel: 1 where K slot and key meet), which is
+// exact, gives lane (c, g) key c at the queries acc_row(., g).
+// MASKED: entries outside the mask are left out again, so that a NaN row (NaN * 0)
+// reaches only keys that its query sees; query row r of the tile sees its keys
+// lo + r < key <= hi + r.
+template <int DT, bool MASKED, bool WIN>
+__device__ __forceinline__ f32x4 tile_colsum(const uint4 (&pa)[2], const uint4 (&sel)[2], const uint4& ones_sel,
+                                             int lo, int hi, int c, int g) {
+    f32x16 t = {};
+    t = mfma16<DT>(pa[0], sel[0], t);
+    t = mfma16<DT>(pa[1], sel[1], t);
+    uint32_t pk[8];
+#pragma unroll
+    for (int j = 0; j < 16; j += 2) {
+        float v[2] = {t[j], t[j + 1]};
+        if constexpr (MASKED) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int r = acc_row(j + u, 32 * g);
+                v[u] = (!WIN || lo + r < c) && c <= hi + r ? v[u] : 0.0f;
+            }
+        }
+        pk[j / 2] = round_pair<DT>(v[0], v[1]);
+    }
+    return tile_sums<DT>(pk, ones_sel);
+}
+
 // A workgroup owns 128 query rows of one query head (wave w: rows 32 w ..),
 // queries resident as the QK^T B operand as in real_rowstats, and streams
 // 64-key stages of K (logits) and Vt (values) through two LDS buffers each.
-template <int DT, int D, bool MAP = false, bool WIN = false>
-__global__ __launch_bounds__(256) void real_output(OutArgs o) {
+// COL: the block's column sums of P, which the scores need; PV: the output.  With
+// both, one pass over the logits serves the two: 32 query and 8 kv heads x 8192 x
+// 128 fp16, kernel trace, 626 us for the output and 436 for the sums by a kernel
+// of their own, which formed every logit again with the keys resident -> 675 and
+// 9 (colsum_blocks).  Without PV, rows in lanes spare the reads of the row
+// statistics from LDS that such a kernel needs: scores of that layer in bf16
+// 855 -> 812 us, at head_dim 256 778 -> 707.
+// The matrix cores, the VALU (exponentials) and LDS reads each have about 220 us
+// of the 675; what is left is how far they overlap.  Waves per SIMD: what LDS
+// leaves (PV), or what registers hold without spills.
+template <int DT, int D, bool COL, bool PV, bool MAP = false, bool WIN = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PV || D > 128 ? 2 : WIN ? 3 : 4))) void
+real_output(OutArgs o) {
     __shared__ __align__(16) char k0buf[RealTile<D>::BUF];
     __shared__ __align__(16) char k1buf[RealTile<D>::BUF];
-    __shared__ __align__(16) char v0buf[VtPlan<D>::BUF];
-    __shared__ __align__(16) char v1buf[VtPlan<D>::BUF];
+    __shared__ __align__(16) char v0buf[PV ? VtPlan<D>::BUF : 16];
+    __shared__ __align__(16) char v1buf[PV ? VtPlan<D>::BUF : 16];
+    __shared__ __align__(16) float csum0[COL ? 256 : 4], csum1[COL ? 256 : 4];  // [wave][key of the stage]
     const RealArgs& a = o.r;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 5, c = lane & 31;
     const int item = xcd_item(a);
     if (item >= a.n_items) return;
-    const int n_blocks = (a.seq + 127) / 128;
+    const int n_blocks = o.qb_n;
     const int grp = a.hq / a.hkv;
     const int hh = item % grp;
     const int rest = item / grp;
-    const int qb = n_blocks - 1 - rest % n_blocks;
+    const int qb = o.qb0 + n_blocks - 1 - rest % n_blocks;
     const int bg = rest / n_blocks;
     const int b = bg / a.hkv, hk = bg - b * a.hkv;
     const int hq = hk * grp + hh;
     const int bhq = b * a.hq + hq;
     const uint16_t* qbase = static_cast<const uint16_t*>(a.q) + (size_t)bhq * a.seq * D;
     const uint16_t* kbase = static_cast<const uint16_t*>(a.k) + ((size_t)b * a.hkv + hk) * a.seq * D;
-    const uint16_t* vt_bh = o.vt + ((size_t)b * a.hkv + hk) * D * o.s64;
+    const uint16_t* vt_bh = PV ? o.vt + ((size_t)b * a.hkv + hk) * D * o.s64 : nullptr;
     const int q0 = qb * 128 + wave * 32;
     const bool live = q0 < a.seq;
     const int my_diag = q0 / 32;
@@ -926,22 +809,58 @@ __global__ __launch_bounds__(256) void real_output(OutArgs o) {
     row_operand<D>(qbase, q0 + c, a.seq, g, qa);
     const size_t stat = (size_t)bhq * a.seq;
     const int qi = min(q0 + c, a.seq - 1);
-    const float nm = a.row_max[stat + qi], rz = a.row_sum[stat + qi];
+    // rows past seq repeat the last one: no probability, so that the column sums leave them out
+    const float nm = a.row_max[stat + qi], rz = q0 + c < a.seq ? a.row_sum[stat + qi] : 0.0f;
     f32x16 oacc[D / 32];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) oacc[db] = f32x16{};
+    const uint4 ones_sel = ones_select<DT>(lane);
+    uint4 sel[2];
+    if constexpr (COL) {
+        constexpr uint32_t one = DT == NQ_F16 ? 0x3C00u : 0x3F80u;
+        uint32_t w[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {  // slots 16 (i / 4) + 8 g + 2 (i % 4) and the next
+            const int p = 16 * (i >> 2) + 8 * g + 2 * (i & 3);
+            w[i] = (slot_key(p) == c ? one : 0u) | (slot_key(p + 1) == c ? one << 16 : 0u);
+        }
+        sel[0] = make_uint4(w[0], w[1], w[2], w[3]);
+        sel[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    }
+    float* const partial = COL ? o.partial + ((size_t)bhq * o.qb_n + (qb - o.qb0)) * o.s64 : nullptr;
+    // one wave's 64 lanes: stage it's column sums, the block's waves in order
+    auto flush = [&](int it, const float* cs) {
+        partial[64 * it + lane] = ((cs[lane] + cs[64 + lane]) + cs[128 + lane]) + cs[192 + lane];
+    };
     const DmaPlan<D> kplan;
     const VtPlan<D> vplan(o.s64);
     tile_dma<D>(kplan, kbase, it_lo * 64, a.seq, k0buf);
-    vt_dma<D>(vplan, vt_bh, it_lo, v0buf);
+    if constexpr (PV) vt_dma<D>(vplan, vt_bh, it_lo, v0buf);
     __builtin_amdgcn_s_waitcnt(kWaitVm0);
     __syncthreads();
-    auto stage = [&](int it, const char* ck, const char* cv, char* nk, char* nv) {
+    auto stage = [&](int it, const char* ck, const char* cv, char* nk, char* nv, float* cs, const float* prev_cs) {
         if (it + 1 < n_it) {
             tile_dma<D>(kplan, kbase, (it + 1) * 64, a.seq, nk);
-            vt_dma<D>(vplan, vt_bh, it + 1, nv);
+            if constexpr (PV) vt_dma<D>(vplan, vt_bh, it + 1, nv);
         }
-        if (live) {
+        // the stage before: its sums are complete since the barrier, and the
+        // store is under way while this stage computes
+        if (COL && it > it_lo && wave == (it & 3)) flush(it - 1, prev_cs);
+        f32x4 col[2] = {};
+        if (live && 2 * it + 1 < my_diag && tile_whole<WIN>(2 * it, my_diag, q0, W)) {
+            // both tiles interior: one basic block, so one tile's matrix work
+            // runs under the other's exponentials
+            f32x16 acc[2];
+            uint4 pa[2][2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) acc[t] = logits_lds_regs<DT, D>(ck + t * 32 * RealTile<D>::ROWB, qa, c, g);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                out_probs<DT, false, MAP>(acc[t], nm, rz, a.scaling, 0, 0, g, pa[t], a.logit_map);
+                if constexpr (COL) col[t] += tile_colsum<DT, false, WIN>(pa[t], sel, ones_sel, 0, 0, c, g);
+                if constexpr (PV) out_pv<DT, D>(pa[t], cv, t, c, g, oacc);
+            }
+        } else if (live) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const int kt = 2 * it + t;
@@ -949,12 +868,23 @@ __global__ __launch_bounds__(256) void real_output(OutArgs o) {
                 if (tile_left<WIN>(kt, q0, W)) continue;
                 const f32x16 acc = logits_lds_regs<DT, D>(ck + t * 32 * RealTile<D>::ROWB, qa, c, g);
                 uint4 pa[2];
-                if (tile_whole<WIN>(kt, my_diag, q0, W))
+                if (tile_whole<WIN>(kt, my_diag, q0, W)) {
                     out_probs<DT, false, MAP>(acc, nm, rz, a.scaling, 0, 0, g, pa, a.logit_map);
-                else
+                    if constexpr (COL) col[t] += tile_colsum<DT, false, WIN>(pa, sel, ones_sel, 0, 0, c, g);
+                } else {
                     out_probs<DT, true, MAP, WIN>(acc, nm, rz, a.scaling, q0 + c - W - 32 * kt, q0 + c - 32 * kt, g,
                                                   pa, a.logit_map);
-                out_pv<DT, D>(pa, cv, t, c, g, oacc);
+                    if constexpr (COL)
+                        col[t] += tile_colsum<DT, true, WIN>(pa, sel, ones_sel, q0 - W - 32 * kt, q0 - 32 * kt, c, g);
+                }
+                if constexpr (PV) out_pv<DT, D>(pa, cv, t, c, g, oacc);
+            }
+        }
+        if constexpr (COL) {  // every wave, also with no tile of the stage
+            if ((lane & 15) < 2) {
+                f32x4* const dst = reinterpret_cast<f32x4*>(&cs[64 * wave + 4 * (lane >> 4) + 16 * (lane & 15)]);
+                dst[0] = col[0];
+                dst[8] = col[1];
             }
         }
         __builtin_amdgcn_s_waitcnt(kWaitVm0);
@@ -962,10 +892,11 @@ __global__ __launch_bounds__(256) void real_output(OutArgs o) {
     };
 #pragma unroll 1
     for (int it = it_lo; it < n_it; it += 2) {
-        stage(it, k0buf, v0buf, k1buf, v1buf);
-        if (it + 1 < n_it) stage(it + 1, k1buf, v1buf, k0buf, v0buf);
+        stage(it, k0buf, v0buf, k1buf, v1buf, csum0, csum1);
+        if (it + 1 < n_it) stage(it + 1, k1buf, v1buf, k0buf, v0buf, csum1, csum0);
     }
-    if (!live) return;
+    if (COL && wave == 0) flush(n_it - 1, ((n_it - 1 - it_lo) & 1) ? csum1 : csum0);
+    if (!PV || !live) return;
     // lane (c, g) holds O[q0 + acc_row(j, g)][32 db + c]
     uint16_t* out = static_cast<uint16_t*>(o.out) + (size_t)bhq * a.seq * D;
 #pragma unroll
@@ -981,6 +912,54 @@ __global__ __launch_bounds__(256) void real_output(OutArgs o) {
                 out[(size_t)qrow * D + 32 * db + c] = h;
             }
         }
+}
+
+// sum plus the column sums of one key (of 64-key stage s) over the launch's query
+// blocks that saw the stage, in order: those from the key's own block on, and
+// under a window those whose first stage (real_output's it_lo) is not past it.
+__device__ __forceinline__ float block_sums(const OutArgs& o, int bh, int s, int key, float sum) {
+    const int lo = max(s / 2, o.qb0);
+    const int hi = min((int)(((int64_t)64 * s + 62 + o.r.window) / 128), o.qb0 + o.qb_n - 1);
+    const float* p = o.partial + (size_t)bh * o.qb_n * o.s64 + key;
+    int qb = lo;
+    for (; qb + 7 <= hi; qb += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(qb + u - o.qb0) * o.s64];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sum += v[u];
+    }
+    for (; qb <= hi; ++qb) sum += p[(size_t)(qb - o.qb0) * o.s64];
+    return sum;
+}
+
+// colsum[bh, key] (ADD: added to) by the launch's query blocks
+template <bool ADD>
+__global__ __launch_bounds__(64) void colsum_blocks(OutArgs o) {
+    const int s = blockIdx.x, bh = blockIdx.y, key = 64 * s + threadIdx.x;
+    const bool in = key < o.r.seq;
+    float* const dst = o.r.colsum + (size_t)bh * o.r.seq + key;
+    const float sum = block_sums(o, bh, s, key, ADD && in ? *dst : 0.0f);
+    if (in) *dst = sum;
+}
+
+// colsum_blocks and head_mean_accumulate of one 64-key stage in one launch, with
+// the same sums: wave w takes heads w, w + 16, ...
+constexpr int kHeadWaves = 16;
+__global__ __launch_bounds__(64 * kHeadWaves) void importance_blocks(OutArgs o) {
+    __shared__ float head[kHeadWaves][64];
+    const RealArgs& a = o.r;
+    const int s = blockIdx.x, b = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int key = 64 * s + lane;
+    float total = 0.0f;
+    for (int h0 = 0; h0 < a.hq; h0 += kHeadWaves) {
+        if (h0 + wave < a.hq) head[wave][lane] = block_sums(o, b * a.hq + h0 + wave, s, key, 0.0f);
+        __syncthreads();
+        if (wave == 0)
+            for (int u = 0; u < kHeadWaves && h0 + u < a.hq; ++u) total += head[u][lane];
+        __syncthreads();
+    }
+    if (wave == 0 && key < a.seq) a.importance[(size_t)b * a.seq + key] += total / (float)a.hq;
 }
 
 // importance[b, i] += mean over heads of colsum[b, h, i], the heads summed in
@@ -1007,82 +986,135 @@ __global__ __launch_bounds__(kHeadMeanThreads) void head_mean_accumulate(const f
     importance[(size_t)b * seq + i] += s / (float)hq;
 }
 
+// Query blocks whose column sums are held at once: all of them up to kPartialBytes
+// (8192 keys of 32 heads: 67 MB), else as many as fit, the launches taking turns.
+constexpr int64_t kPartialBytes = (int64_t)128 << 20;
+
+static int partial_blocks(int64_t bh, int seq) {
+    const int64_t n_blocks = ((int64_t)seq + 127) / 128, s64 = ((int64_t)seq + 63) / 64 * 64;
+    const int64_t fit = kPartialBytes / (bh * s64 * 4);
+    return (int)std::max<int64_t>(1, std::min(fit, n_blocks));
+}
+
+static int64_t partial_bytes(int64_t batch, int64_t q_heads, int seq) {
+    const int64_t bh = batch * q_heads;
+    return partial_blocks(bh, seq) * bh * (((int64_t)seq + 63) / 64 * 64) * 4;
+}
+
+// row maxima, row sums and column sums
+static int64_t stats_bytes(int64_t batch, int64_t q_heads, int64_t seq) {
+    return (batch * q_heads * seq * 4 * 3 + 255) / 256 * 256;
+}
+
+template <int DT, int D, bool COL, bool PV>
+static void launch_output(const OutArgs& o, dim3 grid, hipStream_t st) {
+    if (o.r.logit_map) hipLaunchKernelGGL((real_output<DT, D, COL, PV, true, true>), grid, dim3(256), 0, st, o);
+    else if (o.r.window != kNoWindow) hipLaunchKernelGGL((real_output<DT, D, COL, PV, false, true>), grid, dim3(256), 0, st, o);
+    else hipLaunchKernelGGL((real_output<DT, D, COL, PV>), grid, dim3(256), 0, st, o);
+}
+
+static void launch_head_mean(const RealArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL(head_mean_accumulate, dim3((a.seq + kHeadMeanThreads - 1) / kHeadMeanThreads, a.batch),
+                       dim3(kHeadMeanThreads), 0, st, a.colsum, a.importance, a.hq, a.seq);
+}
+
+// Blocks per key up to which importance_blocks takes the place of colsum_blocks
+// and head_mean_accumulate: one launch fewer where the launches count.
+constexpr int kFusedBlocks = 16;
+
+// Scores (PV: and outputs) of all query blocks, as many at a time as their column sums may take
+template <int DT, int D, bool PV>
+static void launch_blocks(OutArgs o, hipStream_t st) {
+    const int n_blocks = (o.r.seq + 127) / 128, bh = o.r.batch * o.r.hq;
+    const int step = partial_blocks(bh, o.r.seq);
+    const int64_t seen = std::min<int64_t>(n_blocks, o.r.window / 128 + 2);  // blocks that see one key
+    const bool fused = step == n_blocks && seen <= kFusedBlocks;
+    for (int qb0 = 0; qb0 < n_blocks; qb0 += step) {
+        o.qb0 = qb0;
+        o.qb_n = std::min(step, n_blocks - qb0);
+        o.r.n_items = o.qb_n * bh;
+        o.r.per_xcd = (o.r.n_items + 7) / 8;
+        launch_output<DT, D, true, PV>(o, dim3(8 * o.r.per_xcd), st);
+        const dim3 sums(o.s64 / 64, fused ? o.r.batch : bh);
+        if (fused) hipLaunchKernelGGL(importance_blocks, sums, dim3(64 * kHeadWaves), 0, st, o);
+        else if (qb0 == 0) hipLaunchKernelGGL((colsum_blocks<false>), sums, dim3(64), 0, st, o);
+        else hipLaunchKernelGGL((colsum_blocks<true>), sums, dim3(64), 0, st, o);
+    }
+    if (!fused) launch_head_mean(o.r, st);
+}
+
 template <int DT, int D>
-static hipError_t launch_real(const RealArgs& a, hipStream_t st) {
+static hipError_t launch_real(const RealArgs& a, float* partial, hipStream_t st) {
     if constexpr (DT == NQ_F32) {
         const int n_tiles = (a.seq + 31) / 32;
         dim3 grid(n_tiles, a.batch * a.hq);
         hipLaunchKernelGGL((real_sweep<DT, D, 0>), grid, dim3(64), 0, st, a);
         hipLaunchKernelGGL((real_sweep<DT, D, 1>), grid, dim3(64), 0, st, a);
         hipLaunchKernelGGL((real_sweep<DT, D, 2>), grid, dim3(64), 0, st, a);
+        launch_head_mean(a, st);
     } else {
         RealArgs w = a;
         const int n_blocks = (a.seq + 127) / 128;
         w.n_items = n_blocks * a.batch * a.hq;
         w.per_xcd = (w.n_items + 7) / 8;
         dim3 grid(8 * w.per_xcd);
-        if (a.logit_map) {
-            hipLaunchKernelGGL((real_rowstats<DT, D, true, true>), grid, dim3(256), 0, st, w);
-            hipLaunchKernelGGL((real_colsum<DT, D, true, true>), grid, dim3(256), 0, st, w);
-        } else if (a.window != kNoWindow) {
+        if (a.logit_map) hipLaunchKernelGGL((real_rowstats<DT, D, true, true>), grid, dim3(256), 0, st, w);
+        else if (a.window != kNoWindow)
             hipLaunchKernelGGL((real_rowstats<DT, D, false, true>), grid, dim3(256), 0, st, w);
-            hipLaunchKernelGGL((real_colsum<DT, D, false, true>), grid, dim3(256), 0, st, w);
-        } else {
-            hipLaunchKernelGGL((real_rowstats<DT, D>), grid, dim3(256), 0, st, w);
-            hipLaunchKernelGGL((real_colsum<DT, D>), grid, dim3(256), 0, st, w);
-        }
+        else hipLaunchKernelGGL((real_rowstats<DT, D>), grid, dim3(256), 0, st, w);
+        OutArgs o = {};
+        o.r = w;
+        o.partial = partial;
+        o.s64 = (a.seq + 63) / 64 * 64;
+        launch_blocks<DT, D, false>(o, st);
     }
-    hipLaunchKernelGGL(head_mean_accumulate, dim3((a.seq + kHeadMeanThreads - 1) / kHeadMeanThreads, a.batch),
-                       dim3(kHeadMeanThreads), 0, st, a.colsum, a.importance, a.hq, a.seq);
     return hipGetLastError();
 }
 
 template <int DT, int D>
-static hipError_t launch_attention(const RealArgs& a, const void* v, void* out, uint16_t* vt, int s64,
+static hipError_t launch_attention(const RealArgs& a, const void* v, void* out, uint16_t* vt, int s64, float* partial,
                                    bool with_importance, hipStream_t st) {
     RealArgs w = a;
-    const int n_blocks = (a.seq + 127) / 128;
-    w.n_items = n_blocks * a.batch * a.hq;
+    const int n_blocks = (a.seq + 127) / 128, bh = a.batch * a.hq;
+    w.n_items = n_blocks * bh;
     w.per_xcd = (w.n_items + 7) / 8;
     dim3 grid(8 * w.per_xcd);
-    const bool map = a.logit_map != nullptr, win = a.window != kNoWindow;
-    if (map) hipLaunchKernelGGL((real_rowstats<DT, D, true, true>), grid, dim3(256), 0, st, w);
-    else if (win) hipLaunchKernelGGL((real_rowstats<DT, D, false, true>), grid, dim3(256), 0, st, w);
+    if (a.logit_map) hipLaunchKernelGGL((real_rowstats<DT, D, true, true>), grid, dim3(256), 0, st, w);
+    else if (a.window != kNoWindow) hipLaunchKernelGGL((real_rowstats<DT, D, false, true>), grid, dim3(256), 0, st, w);
     else hipLaunchKernelGGL((real_rowstats<DT, D>), grid, dim3(256), 0, st, w);
-    if (with_importance) {
-        if (map) hipLaunchKernelGGL((real_colsum<DT, D, true, true>), grid, dim3(256), 0, st, w);
-        else if (win) hipLaunchKernelGGL((real_colsum<DT, D, false, true>), grid, dim3(256), 0, st, w);
-        else hipLaunchKernelGGL((real_colsum<DT, D>), grid, dim3(256), 0, st, w);
-        hipLaunchKernelGGL(head_mean_accumulate, dim3((a.seq + kHeadMeanThreads - 1) / kHeadMeanThreads, a.batch),
-                           dim3(kHeadMeanThreads), 0, st, a.colsum, a.importance, a.hq, a.seq);
-    }
     hipLaunchKernelGGL((vt_slots_kernel<D>), dim3(s64 / 64, a.batch * a.hkv), dim3(256), 0, st,
                        static_cast<const uint16_t*>(v), vt, a.seq, s64);
     OutArgs o;
     o.r = w;
     o.vt = vt;
     o.out = out;
+    o.partial = partial;
     o.s64 = s64;
-    if (map) hipLaunchKernelGGL((real_output<DT, D, true, true>), grid, dim3(256), 0, st, o);
-    else if (win) hipLaunchKernelGGL((real_output<DT, D, false, true>), grid, dim3(256), 0, st, o);
-    else hipLaunchKernelGGL((real_output<DT, D>), grid, dim3(256), 0, st, o);
+    if (!with_importance) {
+        o.qb0 = 0;
+        o.qb_n = n_blocks;
+        launch_output<DT, D, false, true>(o, grid, st);
+        return hipGetLastError();
+    }
+    launch_blocks<DT, D, true>(o, st);
     return hipGetLastError();
 }
 
 template <int DT>
-static hipError_t dispatch_real_d(int d, const RealArgs& a, hipStream_t st) {
+static hipError_t dispatch_real_d(int d, const RealArgs& a, float* partial, hipStream_t st) {
     switch (d) {
-        case 64: return launch_real<DT, 64>(a, st);
-        case 96: return launch_real<DT, 96>(a, st);
-        case 128: return launch_real<DT, 128>(a, st);
-        default: return launch_real<DT, 256>(a, st);
+        case 64: return launch_real<DT, 64>(a, partial, st);
+        case 96: return launch_real<DT, 96>(a, partial, st);
+        case 128: return launch_real<DT, 128>(a, partial, st);
+        default: return launch_real<DT, 256>(a, partial, st);
     }
 }
 
 }  // namespace nq
 
 extern "C" int64_t nq_score_real_workspace(int32_t batch, int32_t q_heads, int32_t seq) {
-    return (int64_t)batch * q_heads * seq * 4 * 3;
+    if (batch <= 0 || q_heads <= 0 || seq <= 0) return 0;
+    return nq::stats_bytes(batch, q_heads, seq) + nq::partial_bytes(batch, q_heads, seq);
 }
 
 extern "C" int nq_score_real(const void* q, const void* k, int32_t dtype, int32_t batch, int32_t q_heads,
@@ -1119,12 +1151,13 @@ extern "C" int nq_score_real(const void* q, const void* k, int32_t dtype, int32_
     a.scaling = scaling;
     a.window = sliding_window > 0 && sliding_window < kNoWindow ? sliding_window : kNoWindow;
     a.logit_map = logit_map;
+    float* partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + stats_bytes(batch, q_heads, seq));
     hipStream_t st = (hipStream_t)stream;
     hipError_t e;
     switch (dtype) {
-        case NQ_F16: e = dispatch_real_d<NQ_F16>(head_dim, a, st); break;
-        case NQ_BF16: e = dispatch_real_d<NQ_BF16>(head_dim, a, st); break;
-        default: e = dispatch_real_d<NQ_F32>(head_dim, a, st); break;
+        case NQ_F16: e = dispatch_real_d<NQ_F16>(head_dim, a, partial, st); break;
+        case NQ_BF16: e = dispatch_real_d<NQ_BF16>(head_dim, a, partial, st); break;
+        default: e = dispatch_real_d<NQ_F32>(head_dim, a, partial, st); break;
     }
     NQ_CHECK_HIP(e);
     return NQ_OK;
@@ -1133,9 +1166,9 @@ extern "C" int nq_score_real(const void* q, const void* k, int32_t dtype, int32_
 extern "C" int64_t nq_attention_real_workspace(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t seq,
                                                int32_t head_dim) {
     if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || seq <= 0 || head_dim <= 0) return 0;
-    const int64_t stats = (nq_score_real_workspace(batch, q_heads, seq) + 255) / 256 * 256;
+    const int64_t stats = nq::stats_bytes(batch, q_heads, seq);
     const int64_t s64 = ((int64_t)seq + 63) / 64 * 64;
-    return stats + (int64_t)batch * kv_heads * head_dim * s64 * 2;
+    return stats + (int64_t)batch * kv_heads * head_dim * s64 * 2 + nq::partial_bytes(batch, q_heads, seq);
 }
 
 extern "C" int nq_attention_real(const void* q, const void* k, const void* v, int32_t dtype, int32_t batch,
@@ -1173,18 +1206,19 @@ extern "C" int nq_attention_real(const void* q, const void* k, const void* v, in
     a.scaling = scaling;
     a.window = sliding_window > 0 && sliding_window < kNoWindow ? sliding_window : kNoWindow;
     a.logit_map = logit_map;
-    const int64_t stats = (nq_score_real_workspace(batch, q_heads, seq) + 255) / 256 * 256;
+    const int64_t stats = stats_bytes(batch, q_heads, seq);
     uint16_t* vt = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + stats);
     const int s64 = (seq + 63) / 64 * 64;
+    float* partial = reinterpret_cast<float*>(vt + (int64_t)batch * kv_heads * head_dim * s64);
     hipStream_t st = (hipStream_t)stream;
     hipError_t e;
     const bool imp = importance != nullptr;
     if (dtype == NQ_F16)
-        e = head_dim == 64 ? launch_attention<NQ_F16, 64>(a, v, out, vt, s64, imp, st)
-                           : launch_attention<NQ_F16, 128>(a, v, out, vt, s64, imp, st);
+        e = head_dim == 64 ? launch_attention<NQ_F16, 64>(a, v, out, vt, s64, partial, imp, st)
+                           : launch_attention<NQ_F16, 128>(a, v, out, vt, s64, partial, imp, st);
     else
-        e = head_dim == 64 ? launch_attention<NQ_BF16, 64>(a, v, out, vt, s64, imp, st)
-                           : launch_attention<NQ_BF16, 128>(a, v, out, vt, s64, imp, st);
+        e = head_dim == 64 ? launch_attention<NQ_BF16, 64>(a, v, out, vt, s64, partial, imp, st)
+                           : launch_attention<NQ_BF16, 128>(a, v, out, vt, s64, partial, imp, st);
     NQ_CHECK_HIP(e);
     return NQ_OK;
 }
