@@ -14,11 +14,11 @@
 //     the page's bytes (the codes are the B operand, 16 consecutive bytes a lane).
 //     A result tile leaves each lane 4 coordinates of its token, and of the
 //     coordinates D/2 further on: RoPE's pairs, so the merged top stage + forward
-//     RoPE is lane-local.  Rounded to fp16 the tiles are the A operand of
-//     16x16x32 MFMAs with the query heads as columns, their k order matched by the
-//     order the queries are laid out in LDS.  The row scale multiplies the logit, in
-//     fp32, not the key: one rounding per coordinate either way.  bf16 queries take
-//     the keys as two bf16 parts, fp32 queries fp32 FMAs on the unrounded keys.
+//     RoPE is lane-local.  Scaled, rotated and rounded to fp16 -- bit for bit the
+//     keys the page decoder writes -- the tiles are the A operand of 16x16x32 MFMAs
+//     with the query heads as columns, their k order matched by the order the
+//     queries are laid out in LDS.  bf16 queries take the fp16 keys as two bf16
+//     parts (8 + 8 bits hold fp16's 11: exact), fp32 queries fp32 FMAs.
 //  2. Per query head the chunk max x_m of the unscaled logits and
 //     e = exp((x - x_m) / scale_divisor), l = sum e (fixed order); LDS keeps
 //     the weight e * scale_v / 2 per token as an fp16 pair hi + lo.
@@ -192,7 +192,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     constexpr int QOP = QF32 ? G * KM::T * 4 * 2 : KM::T * 64;
     __shared__ __attribute__((aligned(16))) float s_w[kChunk * G];  // [token][head]: logits, then e * scale_v / 2
     __shared__ float s_a[kChunk];       // scale_v / 2 per token
-    __shared__ float s_k[kChunk];       // scale_k h_D / 2 per token
     __shared__ float s_red[4][G];   // per wave: each head's max, then
     __shared__ float s_sum[4][G];   // its sum of exp
     // the query operands until the logits are done, then the waves' value sums
@@ -311,6 +310,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
             for (int s = 0; s < KM::NK; ++s)
 #pragma unroll
                 for (int i = 0; i < KM::W; ++i) kin.c[hf][s][i] = permute(kin.c[hf][s][i]);
+        const float k_scale = (0.5f * f16_bits_to_f32(kin.ks)) * a.hscale;     // token n16's
         float4v la[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};  // two independent chains
         float lf[QF32 ? G : 1] = {};
 #pragma unroll
@@ -336,29 +336,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
                     p[i] = cs + sn;
                 }
             }
-            float x[8];  // coordinates 16 t + 4 kg + i, and those D / 2 on
+            half2v kf[4];  // coordinates 16 t + 4 kg + 0..3, and those D / 2 on, as the page decoder writes them
+            {
+                float x[8];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float lo = (float)y0[i], hi = (float)y1[i];
-                x[i] = __builtin_fmaf(-lo, m[i], hi * p[i]);
-                x[4 + i] = __builtin_fmaf(lo, p[i], hi * m[i]);
+                for (int i = 0; i < 4; ++i) {
+                    const float lo = (float)y0[i] * k_scale, hi = (float)y1[i] * k_scale;
+                    x[i] = __builtin_fmaf(-lo, m[i], hi * p[i]);
+                    x[4 + i] = __builtin_fmaf(lo, p[i], hi * m[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) asm("" : "+v"(x[i]));  // fp32, then fp16: two roundings
+#pragma unroll
+                for (int k = 0; k < 4; ++k) kf[k] = half2v{(__fp16)x[2 * k], (__fp16)x[2 * k + 1]};
             }
             if constexpr (QF16) {
-                u32x4v kf;
+                u32x4v ka;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) asm("" : "+v"(x[i]));  // one packed conversion per pair, not two mixed fmas
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    kf[k] = __builtin_bit_cast(uint32_t, half2v{(__fp16)x[2 * k], (__fp16)x[2 * k + 1]});
-                la[t & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, kf),
+                for (int k = 0; k < 4; ++k) ka[k] = __builtin_bit_cast(uint32_t, kf[k]);
+                la[t & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, ka),
                                                                    __builtin_bit_cast(half8v, s_q[t * 64 + lane]), la[t & 1], 0, 0, 0);
             } else if constexpr (QDT == NQ_BF16) {
                 u32x4v kp[2];  // the key as two bf16 parts
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    kp[0][k] = pk_bf16(x[2 * k], x[2 * k + 1]);
-                    kp[1][k] = pk_bf16(x[2 * k] - __builtin_bit_cast(float, kp[0][k] << 16),
-                                       x[2 * k + 1] - __builtin_bit_cast(float, kp[0][k] & 0xffff0000u));
+                    const float x0 = (float)kf[k].x, x1 = (float)kf[k].y;
+                    kp[0][k] = pk_bf16(x0, x1);
+                    kp[1][k] = pk_bf16(x0 - __builtin_bit_cast(float, kp[0][k] << 16),
+                                       x1 - __builtin_bit_cast(float, kp[0][k] & 0xffff0000u));
                 }
                 const bf16x8v qv = __builtin_bit_cast(bf16x8v, s_q[t * 64 + lane]);
 #pragma unroll
@@ -369,7 +374,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
                 for (int g = 0; g < G; ++g) {
                     const float* qv = reinterpret_cast<const float*>(s_q) + g * D + 32 * t + 8 * kg;
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) lf[g] = __builtin_fmaf(x[i], qv[i], lf[g]);
+                    for (int i = 0; i < 8; ++i)
+                        lf[g] = __builtin_fmaf((float)((i & 1) ? kf[i / 2].y : kf[i / 2].x), qv[i], lf[g]);
                 }
             }
         }
@@ -389,10 +395,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
                 if (n16 < G && tt < rc.n && rc.coff + tt < kChunk) s_w[(rc.coff + tt) * G + n16] = lg[i];
             }
         }
-        if (kg == 0 && n16 < rc.n && rc.coff + n16 < kChunk) {
-            s_a[rc.coff + n16] = 0.5f * f16_bits_to_f32(kin.vs);
-            s_k[rc.coff + n16] = (0.5f * f16_bits_to_f32(kin.ks)) * a.hscale;
-        }
+        if (kg == 0 && n16 < rc.n && rc.coff + n16 < kChunk) s_a[rc.coff + n16] = 0.5f * f16_bits_to_f32(kin.vs);
         rc = rn;
         rn = r2;
         kin = knext;
@@ -406,11 +409,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     __shared__ float s_amax[4];
     {
         float v = -__builtin_inff();
-        for (int i = threadIdx.x; i < n_tok * G; i += 256) {
-            const float x = s_w[i] * s_k[i / G];  // read again by this thread below
-            s_w[i] = x;
-            v = __builtin_fmaxf(v, x);
-        }
+        for (int i = threadIdx.x; i < n_tok * G; i += 256) v = __builtin_fmaxf(v, s_w[i]);
 #pragma unroll
         for (int o = 32; o >= G; o >>= 1) v = __builtin_fmaxf(v, __shfl_xor(v, o, 64));
         if (lane < G) s_red[wave][lane] = v;

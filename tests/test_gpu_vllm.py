@@ -390,3 +390,40 @@ def test_compress_pages_takes_positions_of_any_kind():
             assert torch.equal(getattr(many, name), getattr(one, name)), name
     with pytest.raises(ValueError, match="non-negative"):
         comp.compress_pages([(work[0][0], work[0][1], torch.arange(-1, 6))])
+
+
+@pytest.mark.parametrize("d,group,qdt", [(64, 8, torch.float16), (128, 8, torch.float16), (128, 4, torch.float16),
+                                         (256, 1, torch.float16), (64, 4, torch.bfloat16), (128, 4, torch.bfloat16),
+                                         (256, 2, torch.bfloat16), (64, 1, torch.float32), (128, 2, torch.float32),
+                                         (256, 4, torch.float32)])
+def test_paged_forward_takes_the_page_decoders_keys(d, group, qdt):
+    """The keys of decode attention are the fp16 keys that decompress_pages returns.
+
+    Queries orthogonal to a row's keys and 2000 long per coordinate: the logits are what
+    the keys' rounding leaves, times 2000 (a key rounded elsewhere moves a logit by 0.2)."""
+    from nexusquant_amd.vllm_backend import CompressedPage, NexusQuantKVCompressor, NexusQuantPagedAttention
+    print(f"[gpu] decoder's keys d={d} group={group} {qdt}", flush=True)
+    kv, n = 2, 15
+    g = torch.Generator(device=DEV).manual_seed(d + group)
+    comp = NexusQuantKVCompressor(head_dim=d, bits=3, rope_base=10000.0)
+    attn = NexusQuantPagedAttention(comp)
+    page = comp.compress_page(torch.randn(kv, n, d, device=DEV, generator=g).half(),
+                              torch.randn(kv, n, d, device=DEV, generator=g).half(),
+                              torch.arange(n, dtype=torch.int32) + 5000)
+    k, v = (t.double() for t in comp.decompress_pages([page])[0])
+    q = torch.empty(1, kv * group, d, dtype=torch.float64, device=DEV)
+    for h in range(kv * group):
+        x = torch.randn(d, dtype=torch.float64, device=DEV, generator=g)
+        basis = torch.linalg.qr(k[h // group].T.cpu())[0].to(DEV)
+        q[0, h] = 2000 * (x - basis @ (basis.T @ x))
+    q = q.to(qdt)
+    got = attn.forward(q, {0: page}, {0: page}, [[0]], torch.tensor([n]))
+    for h in range(kv * group):
+        kh, qh = k[h // group], q[0, h].double()
+        want = torch.softmax(kh @ qh / math.sqrt(d), 0) @ v[h // group]
+        # fp32 sums of d exact products, rounded at random: 4 sqrt(d) 2^-24 of the products' sum
+        # in a logit, as much relatively in a weight; the output rounded to fp16 and to the query's type
+        logit = 4 * math.sqrt(d) * 2.0 ** -24 * float((kh.abs() @ qh.abs()).max()) / math.sqrt(d)
+        tol = logit + (2.0 ** -8 if qdt == torch.bfloat16 else 2.0 ** -10)
+        err = float((got[0, h].double() - want).norm() / want.norm())
+        assert err <= tol, (h, err, tol)
