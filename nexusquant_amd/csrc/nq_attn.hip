@@ -180,10 +180,12 @@ __device__ __forceinline__ float wave_sum(float v) {
 // MT: the merged RoPE tables are given (else they are formed from cos and sin;
 // a template, because a branch between an MFMA and the first use of its result
 // hides the wait that the result needs from the compiler's hazard checks).
-// Registers: fp16 queries fit 4 waves per SIMD at D = 128 (121 VGPRs), the others
-// would spill there and take 3, fp32 queries of 4 heads 2.
+// Registers: 4 waves per SIMD fit at D = 128 (113..123 VGPRs), 2 at 256 (177..220); no
+// variant spills.  fp32 queries, 8 kv heads x 32768 tokens, us against the form that
+// decoded the keys on the vector ALUs: D = 128 with 2 and 4 heads 31.1 -> 30.8 and 34.9 ->
+// 34.3, D = 256 49.8 -> 45.3 and 56.7 -> 53.8 (with spills 37.9, 29.6, 94 and 207).
 template <int D, int G, int QDT, bool MT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : D == 256 || (QDT == NQ_F32 && G >= 4) ? 2 : QDT == NQ_F16 ? 4 : 3))) void paged_attn_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 4 : 2))) void paged_attn_kernel(
     AttnArgs a) {
     using KM = KeyMfma<D>;
     constexpr bool QF16 = QDT == NQ_F16;
@@ -372,10 +374,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
             } else {
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
-                    const float* qv = reinterpret_cast<const float*>(s_q) + g * D + 32 * t + 8 * kg;
+                    const float4v* qv = reinterpret_cast<const float4v*>(s_q) + 2 * (g * D / 8 + 4 * t + kg);
+                    const float4v q0 = qv[0], q1 = qv[1];
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
-                        lf[g] = __builtin_fmaf((float)((i & 1) ? kf[i / 2].y : kf[i / 2].x), qv[i], lf[g]);
+                        lf[g] = __builtin_fmaf((float)((i & 1) ? kf[i / 2].y : kf[i / 2].x), i < 4 ? q0[i & 3] : q1[i & 3], lf[g]);
+                    // summed here, two heads at a time: sunk to the stores below, every head's
+                    // queries of the unit would be in registers at once (up to 840 bytes a lane spilled)
+                    if (g & 1) asm volatile("" : "+v"(lf[g - 1]), "+v"(lf[g]));
+                    else if (g == G - 1) asm volatile("" : "+v"(lf[g]));
                 }
             }
         }
