@@ -427,3 +427,30 @@ def test_paged_forward_takes_the_page_decoders_keys(d, group, qdt):
         tol = logit + (2.0 ** -8 if qdt == torch.bfloat16 else 2.0 ** -10)
         err = float((got[0, h].double() - want).norm() / want.norm())
         assert err <= tol, (h, err, tol)
+
+
+@pytest.mark.parametrize("d,group,qdt", [(128, 4, torch.float16), (128, 4, torch.bfloat16), (64, 2, torch.float32)])
+def test_paged_forward_row_alone_and_in_a_batch(d, group, qdt):
+    """A row planned alone is cut at 64 tokens, among long rows at 512: the outputs agree to
+    one rounding of the output."""
+    from nexusquant_amd.vllm_backend import NexusQuantKVCompressor, NexusQuantPagedAttention
+    print(f"[gpu] row alone and in a batch d={d} group={group} {qdt}", flush=True)
+    kv, size = 2, 1024
+    g = torch.Generator(device=DEV).manual_seed(d + group)
+    comp = NexusQuantKVCompressor(head_dim=d, bits=3, rope_base=500000.0)
+    attn = NexusQuantPagedAttention(comp)
+    work = [(torch.randn(kv, size, d, device=DEV, generator=g).half(), torch.randn(kv, size, d, device=DEV, generator=g).half(),
+             torch.arange(size, dtype=torch.int32) + size * i) for i in range(4)]
+    cache = dict(enumerate(comp.compress_pages(work)))
+    tables = [[0, 1]] + [[0, 1, 2, 3]] * 32
+    ctx = [1500] + [4096] * 32
+    q = torch.randn(33, kv * group, d, device=DEV, generator=g).to(qdt)
+    alone, batch = attn.plan(cache, tables[:1], ctx[:1]), attn.plan(cache, tables, ctx)
+    assert alone.n_chunks == -(-1500 // 64) and batch.n_chunks == 3 + 32 * 8
+    a, b = attn.run(alone, q[:1])[0].double(), attn.run(batch, q)[0].double()
+    # weights: x and the chunk's max are rounded to 2^-24 and differ by less than 2^4, exp to a
+    # few ulp: 2^-18 of a weight; the output's rounding to fp16 (2^-11) and bf16 (2^-9) may fall
+    # either way
+    vmax = max(float(p[1].abs().max()) for p in comp.decompress_pages(list(cache.values())))
+    ulp = 2.0 ** -8 + 2.0 ** -10 if qdt == torch.bfloat16 else 2.0 ** -10
+    assert bool(((a - b).abs() <= ulp * a.abs() + 2.0 ** -17 * vmax).all())
