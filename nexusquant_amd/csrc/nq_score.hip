@@ -221,8 +221,6 @@ template <int D>
 struct RealTile {
     static constexpr int ROWB = 2 * D + 16;          // padded LDS row bytes
     static constexpr int ROWS = 64;                  // rows per LDS stage (two 32-row MFMA blocks)
-    static constexpr int UNITS = ROWS * D / 8;       // 16-byte units per stage
-    static constexpr int PER_THREAD = (UNITS + 255) / 256;
     static constexpr int KS = D / 16;                // MFMA K steps
     static constexpr int BUF = ROWS * ROWB;
 };
@@ -305,14 +303,18 @@ __device__ __forceinline__ void tile_dma(const DmaPlan<D>& plan, const uint16_t*
     }
 }
 
-// 32x32 logits: A (queries) from 32 LDS rows, B (keys) from registers.
-template <int DT, int D>
-__device__ __forceinline__ f32x16 logits_lds_regs(const char* lds, const uint4 (&b)[RealTile<D>::KS], int c, int g) {
+// 32x32 logits of 32 keys in LDS rows and 32 queries in registers.  Keys are the A
+// operand: lane (c, g) gets query c at the keys acc_row(., g).  T: queries are, and
+// it gets key c at the queries acc_row(., g).
+template <int DT, int D, bool T = false>
+__device__ __forceinline__ f32x16 logits_lds_regs(const char* lds, const uint4 (&q)[RealTile<D>::KS], int c, int g) {
     f32x16 acc = {};
     const char* row = lds + c * RealTile<D>::ROWB + 16 * g;
 #pragma unroll
-    for (int s = 0; s < RealTile<D>::KS; ++s)
-        acc = mfma16<DT>(*reinterpret_cast<const uint4*>(row + 32 * s), b[s], acc);
+    for (int s = 0; s < RealTile<D>::KS; ++s) {
+        const uint4 k = *reinterpret_cast<const uint4*>(row + 32 * s);
+        acc = T ? mfma16<DT>(q[s], k, acc) : mfma16<DT>(k, q[s], acc);
+    }
     return acc;
 }
 
@@ -689,10 +691,15 @@ struct OutArgs {
     RealArgs r;
     const uint16_t* vt;  // [batch * hkv, D, s64]
     void* out;           // [batch, hq, seq, D] in the model dtype
-    float* partial;      // COL: [batch * hq, qb_n, s64] column sums of one 128-query block each
-    int32_t s64;
+    float* partial;      // COL: [batch * hq, qb_n, ps] column sums of one 128-query block each, from
+                         // the first stage it sees on
+    int32_t s64, ps;
     int32_t qb0, qb_n;   // the launch's query blocks [qb0, qb0 + qb_n)
+    int32_t segs;        // without PV: workgroups that share a block's stages
 };
+
+// First 64-key stage that 128-query block qb sees under window W.
+__device__ __forceinline__ int first_stage(int qb, int W) { return max(qb * 128 - W + 1, 0) / 64; }
 
 // Rounded probabilities of one 32 x 32 logit tile for this lane's query (nm,
 // rz its row statistics), packed for the two 16-deep K steps of P V.
@@ -761,21 +768,47 @@ __device__ __forceinline__ f32x4 tile_colsum(const uint4 (&pa)[2], const uint4 (
     return tile_sums<DT>(pk, ones_sel);
 }
 
+// Column sums of one tile of logits whose lanes hold key c at the queries
+// acc_row(., g), nm and rz their row statistics: the probabilities of out_probs,
+// bit for bit, where tile_colsum's transposition puts them.  MASKED as there.
+template <int DT, bool MASKED, bool MAP, bool WIN>
+__device__ __forceinline__ f32x4 key_colsum(const f32x16& acc, const float (&nm)[16], const float (&rz)[16], float scaling,
+                                            const uint4& ones_sel, int lo, int hi, int c, int g, const uint16_t* map) {
+    uint32_t pk[8];
+#pragma unroll
+    for (int j = 0; j < 16; j += 2) {
+        float x[2], p[2];
+        exp_args2<DT, MAP>(acc[j], acc[j + 1], scaling, nm[j], nm[j + 1], x[0], x[1], map);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            p[u] = __builtin_amdgcn_exp2f(x[u]) * rz[j + u];
+            if constexpr (MASKED) {
+                const int r = acc_row(j + u, 32 * g);
+                p[u] = (!WIN || lo + r < c) && c <= hi + r ? p[u] : 0.0f;
+            }
+        }
+        pk[j / 2] = round_pair<DT>(p[0], p[1]);
+    }
+    return tile_sums<DT>(pk, ones_sel);
+}
+
+// Waves per SIMD, and workgroups per CU: what LDS leaves (PV) or what registers hold
+// without spills.
+constexpr int output_waves(int D, bool PV, bool WIN) { return PV || D > 128 ? 2 : WIN || D > 64 ? 3 : 4; }
+
 // A workgroup owns 128 query rows of one query head (wave w: rows 32 w ..),
-// queries resident as the QK^T B operand as in real_rowstats, and streams
+// queries resident as an operand of QK^T as in real_rowstats, and streams
 // 64-key stages of K (logits) and Vt (values) through two LDS buffers each.
 // COL: the block's column sums of P, which the scores need; PV: the output.  With
 // both, one pass over the logits serves the two: 32 query and 8 kv heads x 8192 x
 // 128 fp16, kernel trace, 626 us for the output and 436 for the sums by a kernel
 // of their own, which formed every logit again with the keys resident -> 675 and
-// 9 (colsum_blocks).  Without PV, rows in lanes spare the reads of the row
-// statistics from LDS that such a kernel needs: scores of that layer in bf16
-// 855 -> 812 us, at head_dim 256 778 -> 707.
-// The matrix cores, the VALU (exponentials) and LDS reads each have about 220 us
-// of the 675; what is left is how far they overlap.  Waves per SIMD: what LDS
-// leaves (PV), or what registers hold without spills.
+// 9 (colsum_blocks).  Without PV the operands are swapped: a lane then holds one key's
+// logits at 16 queries, whose statistics stay in its registers, and nothing is
+// transposed (16 heads x 4096 x 64 fp16 with window 1024, kernel: 34 us transposed, 31
+// with the keys resident, 29 so and with a block's stages shared).
 template <int DT, int D, bool COL, bool PV, bool MAP = false, bool WIN = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PV || D > 128 ? 2 : WIN ? 3 : 4))) void
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(output_waves(D, PV, WIN)))) void
 real_output(OutArgs o) {
     __shared__ __align__(16) char k0buf[RealTile<D>::BUF];
     __shared__ __align__(16) char k1buf[RealTile<D>::BUF];
@@ -789,7 +822,9 @@ real_output(OutArgs o) {
     const int n_blocks = o.qb_n;
     const int grp = a.hq / a.hkv;
     const int hh = item % grp;
-    const int rest = item / grp;
+    int rest = item / grp;
+    const int seg = PV ? 0 : rest % o.segs;
+    if constexpr (!PV) rest /= o.segs;
     const int qb = o.qb0 + n_blocks - 1 - rest % n_blocks;
     const int bg = rest / n_blocks;
     const int b = bg / a.hkv, hk = bg - b * a.hkv;
@@ -802,21 +837,30 @@ real_output(OutArgs o) {
     const bool live = q0 < a.seq;
     const int my_diag = q0 / 32;
     const int last_key = min(qb * 128 + 127, a.seq - 1);
-    const int n_it = last_key / 64 + 1;
     const int W = WIN ? a.window : kNoWindow;
-    const int it_lo = WIN ? max(qb * 128 - W + 1, 0) / 64 : 0;
+    const int it_first = WIN ? first_stage(qb, W) : 0, n_all = last_key / 64 + 1 - it_first;
+    const int it_lo = PV ? it_first : it_first + n_all * seg / o.segs;
+    const int n_it = PV ? it_first + n_all : it_first + n_all * (seg + 1) / o.segs;
+    if (it_lo >= n_it) return;  // more workgroups than stages
     uint4 qa[RealTile<D>::KS];
     row_operand<D>(qbase, q0 + c, a.seq, g, qa);
     const size_t stat = (size_t)bhq * a.seq;
-    const int qi = min(q0 + c, a.seq - 1);
-    // rows past seq repeat the last one: no probability, so that the column sums leave them out
-    const float nm = a.row_max[stat + qi], rz = q0 + c < a.seq ? a.row_sum[stat + qi] : 0.0f;
+    // the row statistics of this lane's query, or without PV of its 16.  Rows past seq
+    // repeat the last one: no probability, so that the column sums leave them out
+    constexpr int NS = PV ? 1 : 16;
+    float nm[NS], rz[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+        const int q = q0 + (PV ? c : acc_row(j, 32 * g)), qi = min(q, a.seq - 1);
+        nm[j] = a.row_max[stat + qi];
+        rz[j] = q < a.seq ? a.row_sum[stat + qi] : 0.0f;
+    }
     f32x16 oacc[D / 32];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) oacc[db] = f32x16{};
     const uint4 ones_sel = ones_select<DT>(lane);
     uint4 sel[2];
-    if constexpr (COL) {
+    if constexpr (COL && PV) {
         constexpr uint32_t one = DT == NQ_F16 ? 0x3C00u : 0x3F80u;
         uint32_t w[8];
 #pragma unroll
@@ -827,10 +871,10 @@ real_output(OutArgs o) {
         sel[0] = make_uint4(w[0], w[1], w[2], w[3]);
         sel[1] = make_uint4(w[4], w[5], w[6], w[7]);
     }
-    float* const partial = COL ? o.partial + ((size_t)bhq * o.qb_n + (qb - o.qb0)) * o.s64 : nullptr;
+    float* const partial = COL ? o.partial + ((size_t)bhq * o.qb_n + (qb - o.qb0)) * o.ps : nullptr;
     // one wave's 64 lanes: stage it's column sums, the block's waves in order
     auto flush = [&](int it, const float* cs) {
-        partial[64 * it + lane] = ((cs[lane] + cs[64 + lane]) + cs[128 + lane]) + cs[192 + lane];
+        partial[64 * (it - it_first) + lane] = ((cs[lane] + cs[64 + lane]) + cs[128 + lane]) + cs[192 + lane];
     };
     const DmaPlan<D> kplan;
     const VtPlan<D> vplan(o.s64);
@@ -851,14 +895,18 @@ real_output(OutArgs o) {
             // both tiles interior: one basic block, so one tile's matrix work
             // runs under the other's exponentials
             f32x16 acc[2];
-            uint4 pa[2][2];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) acc[t] = logits_lds_regs<DT, D>(ck + t * 32 * RealTile<D>::ROWB, qa, c, g);
+            for (int t = 0; t < 2; ++t) acc[t] = logits_lds_regs<DT, D, !PV>(ck + t * 32 * RealTile<D>::ROWB, qa, c, g);
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                out_probs<DT, false, MAP>(acc[t], nm, rz, a.scaling, 0, 0, g, pa[t], a.logit_map);
-                if constexpr (COL) col[t] += tile_colsum<DT, false, WIN>(pa[t], sel, ones_sel, 0, 0, c, g);
-                if constexpr (PV) out_pv<DT, D>(pa[t], cv, t, c, g, oacc);
+                if constexpr (PV) {
+                    uint4 pa[2];
+                    out_probs<DT, false, MAP>(acc[t], nm[0], rz[0], a.scaling, 0, 0, g, pa, a.logit_map);
+                    if constexpr (COL) col[t] += tile_colsum<DT, false, WIN>(pa, sel, ones_sel, 0, 0, c, g);
+                    out_pv<DT, D>(pa, cv, t, c, g, oacc);
+                } else {
+                    col[t] += key_colsum<DT, false, MAP, WIN>(acc[t], nm, rz, a.scaling, ones_sel, 0, 0, c, g, a.logit_map);
+                }
             }
         } else if (live) {
 #pragma unroll
@@ -866,18 +914,24 @@ real_output(OutArgs o) {
                 const int kt = 2 * it + t;
                 if (kt > my_diag) break;
                 if (tile_left<WIN>(kt, q0, W)) continue;
-                const f32x16 acc = logits_lds_regs<DT, D>(ck + t * 32 * RealTile<D>::ROWB, qa, c, g);
-                uint4 pa[2];
-                if (tile_whole<WIN>(kt, my_diag, q0, W)) {
-                    out_probs<DT, false, MAP>(acc, nm, rz, a.scaling, 0, 0, g, pa, a.logit_map);
-                    if constexpr (COL) col[t] += tile_colsum<DT, false, WIN>(pa, sel, ones_sel, 0, 0, c, g);
+                const f32x16 acc = logits_lds_regs<DT, D, !PV>(ck + t * 32 * RealTile<D>::ROWB, qa, c, g);
+                const int lo = q0 - W - 32 * kt, hi = q0 - 32 * kt;  // of the tile's first query
+                const bool whole = tile_whole<WIN>(kt, my_diag, q0, W);
+                if constexpr (PV) {
+                    uint4 pa[2];
+                    if (whole) {
+                        out_probs<DT, false, MAP>(acc, nm[0], rz[0], a.scaling, 0, 0, g, pa, a.logit_map);
+                        if constexpr (COL) col[t] += tile_colsum<DT, false, WIN>(pa, sel, ones_sel, 0, 0, c, g);
+                    } else {
+                        out_probs<DT, true, MAP, WIN>(acc, nm[0], rz[0], a.scaling, lo + c, hi + c, g, pa, a.logit_map);
+                        if constexpr (COL) col[t] += tile_colsum<DT, true, WIN>(pa, sel, ones_sel, lo, hi, c, g);
+                    }
+                    out_pv<DT, D>(pa, cv, t, c, g, oacc);
+                } else if (whole) {
+                    col[t] += key_colsum<DT, false, MAP, WIN>(acc, nm, rz, a.scaling, ones_sel, 0, 0, c, g, a.logit_map);
                 } else {
-                    out_probs<DT, true, MAP, WIN>(acc, nm, rz, a.scaling, q0 + c - W - 32 * kt, q0 + c - 32 * kt, g,
-                                                  pa, a.logit_map);
-                    if constexpr (COL)
-                        col[t] += tile_colsum<DT, true, WIN>(pa, sel, ones_sel, q0 - W - 32 * kt, q0 - 32 * kt, c, g);
+                    col[t] += key_colsum<DT, true, MAP, WIN>(acc, nm, rz, a.scaling, ones_sel, lo, hi, c, g, a.logit_map);
                 }
-                if constexpr (PV) out_pv<DT, D>(pa, cv, t, c, g, oacc);
             }
         }
         if constexpr (COL) {  // every wave, also with no tile of the stage
@@ -916,20 +970,21 @@ real_output(OutArgs o) {
 
 // sum plus the column sums of one key (of 64-key stage s) over the launch's query
 // blocks that saw the stage, in order: those from the key's own block on, and
-// under a window those whose first stage (real_output's it_lo) is not past it.
+// under a window those whose first stage is not past it.
 __device__ __forceinline__ float block_sums(const OutArgs& o, int bh, int s, int key, float sum) {
     const int lo = max(s / 2, o.qb0);
     const int hi = min((int)(((int64_t)64 * s + 62 + o.r.window) / 128), o.qb0 + o.qb_n - 1);
-    const float* p = o.partial + (size_t)bh * o.qb_n * o.s64 + key;
-    int qb = lo;
-    for (; qb + 7 <= hi; qb += 8) {
+    const float* p = o.partial + (size_t)bh * o.qb_n * o.ps + key;
+    for (int qb = lo; qb <= hi; qb += 8) {
         float v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(qb + u - o.qb0) * o.s64];
+        for (int u = 0; u < 8; ++u) {
+            const int x = min(qb + u, hi);
+            v[u] = p[(int64_t)(x - o.qb0) * o.ps - 64 * first_stage(x, o.r.window)];
+        }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) sum += v[u];
+        for (int u = 0; u < 8; ++u) sum += qb + u <= hi ? v[u] : 0.0f;
     }
-    for (; qb <= hi; ++qb) sum += p[(size_t)(qb - o.qb0) * o.s64];
     return sum;
 }
 
@@ -944,13 +999,15 @@ __global__ __launch_bounds__(64) void colsum_blocks(OutArgs o) {
 }
 
 // colsum_blocks and head_mean_accumulate of one 64-key stage in one launch, with
-// the same sums: wave w takes heads w, w + 16, ...
+// the same sums: a wave per head, up to 16, then every 16th head.
 constexpr int kHeadWaves = 16;
 __global__ __launch_bounds__(64 * kHeadWaves) void importance_blocks(OutArgs o) {
     __shared__ float head[kHeadWaves][64];
     const RealArgs& a = o.r;
     const int s = blockIdx.x, b = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int key = 64 * s + lane;
+    float* const imp = a.importance + (size_t)b * a.seq + min(key, a.seq - 1);
+    const float before = *imp;
     float total = 0.0f;
     for (int h0 = 0; h0 < a.hq; h0 += kHeadWaves) {
         if (h0 + wave < a.hq) head[wave][lane] = block_sums(o, b * a.hq + h0 + wave, s, key, 0.0f);
@@ -959,7 +1016,7 @@ __global__ __launch_bounds__(64 * kHeadWaves) void importance_blocks(OutArgs o) 
             for (int u = 0; u < kHeadWaves && h0 + u < a.hq; ++u) total += head[u][lane];
         __syncthreads();
     }
-    if (wave == 0 && key < a.seq) a.importance[(size_t)b * a.seq + key] += total / (float)a.hq;
+    if (wave == 0 && key < a.seq) *imp = before + total / (float)a.hq;
 }
 
 // importance[b, i] += mean over heads of colsum[b, h, i], the heads summed in
@@ -988,17 +1045,23 @@ __global__ __launch_bounds__(kHeadMeanThreads) void head_mean_accumulate(const f
 
 // Query blocks whose column sums are held at once: all of them up to kPartialBytes
 // (8192 keys of 32 heads: 67 MB), else as many as fit, the launches taking turns.
+// A launch that forms the output too wants rounds of kOutBlocks workgroups, two for
+// each CU, and may hold up to kOutputBytes for the first (131072 keys: 268 MB); past
+// that (262144 keys) the sums take a pass of their own.  32 query and 8 kv heads x 131072 x 128
+// bf16: 319 ms with the 256 workgroups that 128 MB hold, 278 so, 317 with launches of
+// one and a half rounds; 351 with a pass of their own for the sums.
 constexpr int64_t kPartialBytes = (int64_t)128 << 20;
+constexpr int64_t kOutputBytes = (int64_t)512 << 20;
+constexpr int64_t kOutBlocks = 512;
 
-static int partial_blocks(int64_t bh, int seq) {
-    const int64_t n_blocks = ((int64_t)seq + 127) / 128, s64 = ((int64_t)seq + 63) / 64 * 64;
-    const int64_t fit = kPartialBytes / (bh * s64 * 4);
-    return (int)std::max<int64_t>(1, std::min(fit, n_blocks));
-}
+static int64_t padded_keys(int64_t seq) { return (seq + 63) / 64 * 64; }
+static int64_t out_round(int64_t bh) { return std::max<int64_t>(1, kOutBlocks / bh); }
 
-static int64_t partial_bytes(int64_t batch, int64_t q_heads, int seq) {
-    const int64_t bh = batch * q_heads;
-    return partial_blocks(bh, seq) * bh * (((int64_t)seq + 63) / 64 * 64) * 4;
+static int64_t partial_bytes(int64_t bh, int64_t seq, bool output) {
+    const int64_t n_blocks = (seq + 127) / 128, block = bh * padded_keys(seq) * 4;
+    int64_t n = std::max<int64_t>(1, kPartialBytes / block);
+    if (output && out_round(bh) * block <= kOutputBytes) n = std::max(n, out_round(bh));
+    return std::min(n, n_blocks) * block;
 }
 
 // row maxima, row sums and column sums
@@ -1022,21 +1085,59 @@ static void launch_head_mean(const RealArgs& a, hipStream_t st) {
 // and head_mean_accumulate: one launch fewer where the launches count.
 constexpr int kFusedBlocks = 16;
 
+// Workgroups that share a block's stages when only its sums are formed: one once the
+// blocks fill the chip twice (slots: workgroups that are resident at once), else the
+// number with the least rounds x stages, counting half a round for the last one and
+// two stages for a workgroup's own loads.  Whole calls, us, one workgroup a block ->
+// this: 8 heads x 500 keys x 128 fp16 29 -> 21, x 2000 82 -> 52; 16 x 4096 x 64 126 ->
+// 101, with window 1024 61 -> 56; ms, 8 x 131072 x 64 bf16 56.5 -> 39.9.
+static int block_segments(int64_t blocks, int64_t stages, int slots) {
+    if (blocks >= 2 * slots) return 1;
+    int best = 1;
+    double least = 0.0;
+    for (int n = 1; n <= 64 && n <= std::max<int64_t>(1, stages / 2); ++n) {
+        const double t = ((double)blocks * n / slots + 0.5) * ((double)stages / n + 2.0);
+        if (n == 1 || t < least) {
+            best = n;
+            least = t;
+        }
+    }
+    return best;
+}
+
 // Scores (PV: and outputs) of all query blocks, as many at a time as their column sums may take
 template <int DT, int D, bool PV>
 static void launch_blocks(OutArgs o, hipStream_t st) {
     const int n_blocks = (o.r.seq + 127) / 128, bh = o.r.batch * o.r.hq;
-    const int step = partial_blocks(bh, o.r.seq);
+    // stages that a block sees, at most: 2 qb + 2 - first_stage(qb)
+    const int64_t stages = std::min<int64_t>(o.s64 / 64, 2 + ((int64_t)o.r.window + 62) / 64);
+    o.ps = (int32_t)(64 * stages);
+    const int64_t held = partial_bytes(bh, o.r.seq, PV) / ((int64_t)bh * o.ps * 4);
+    int step = (int)std::min<int64_t>(held, n_blocks);
+    if constexpr (PV) {
+        const int round = (int)out_round(bh);
+        if (step < std::min(round, n_blocks)) {
+            o.qb0 = 0;
+            o.qb_n = n_blocks;
+            launch_output<DT, D, false, true>(o, dim3(8 * o.r.per_xcd), st);
+            launch_blocks<DT, D, false>(o, st);
+            return;
+        }
+        if (step < n_blocks) step = step / round * round;
+    }
     const int64_t seen = std::min<int64_t>(n_blocks, o.r.window / 128 + 2);  // blocks that see one key
     const bool fused = step == n_blocks && seen <= kFusedBlocks;
+    const int slots = 256 * output_waves(D, PV, o.r.window != kNoWindow || o.r.logit_map);
     for (int qb0 = 0; qb0 < n_blocks; qb0 += step) {
         o.qb0 = qb0;
         o.qb_n = std::min(step, n_blocks - qb0);
-        o.r.n_items = o.qb_n * bh;
+        const int groups = o.qb_n * bh;
+        o.segs = PV ? 1 : block_segments(groups, stages, slots);
+        o.r.n_items = groups * o.segs;
         o.r.per_xcd = (o.r.n_items + 7) / 8;
         launch_output<DT, D, true, PV>(o, dim3(8 * o.r.per_xcd), st);
         const dim3 sums(o.s64 / 64, fused ? o.r.batch : bh);
-        if (fused) hipLaunchKernelGGL(importance_blocks, sums, dim3(64 * kHeadWaves), 0, st, o);
+        if (fused) hipLaunchKernelGGL(importance_blocks, sums, dim3(64 * std::min(o.r.hq, kHeadWaves)), 0, st, o);
         else if (qb0 == 0) hipLaunchKernelGGL((colsum_blocks<false>), sums, dim3(64), 0, st, o);
         else hipLaunchKernelGGL((colsum_blocks<true>), sums, dim3(64), 0, st, o);
     }
@@ -1114,7 +1215,7 @@ static hipError_t dispatch_real_d(int d, const RealArgs& a, float* partial, hipS
 
 extern "C" int64_t nq_score_real_workspace(int32_t batch, int32_t q_heads, int32_t seq) {
     if (batch <= 0 || q_heads <= 0 || seq <= 0) return 0;
-    return nq::stats_bytes(batch, q_heads, seq) + nq::partial_bytes(batch, q_heads, seq);
+    return nq::stats_bytes(batch, q_heads, seq) + nq::partial_bytes((int64_t)batch * q_heads, seq, false);
 }
 
 extern "C" int nq_score_real(const void* q, const void* k, int32_t dtype, int32_t batch, int32_t q_heads,
@@ -1167,8 +1268,8 @@ extern "C" int64_t nq_attention_real_workspace(int32_t batch, int32_t q_heads, i
                                                int32_t head_dim) {
     if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || seq <= 0 || head_dim <= 0) return 0;
     const int64_t stats = nq::stats_bytes(batch, q_heads, seq);
-    const int64_t s64 = ((int64_t)seq + 63) / 64 * 64;
-    return stats + (int64_t)batch * kv_heads * head_dim * s64 * 2 + nq::partial_bytes(batch, q_heads, seq);
+    const int64_t vt = (int64_t)batch * kv_heads * head_dim * nq::padded_keys(seq) * 2;
+    return stats + vt + nq::partial_bytes((int64_t)batch * q_heads, seq, true);
 }
 
 extern "C" int nq_attention_real(const void* q, const void* k, const void* v, int32_t dtype, int32_t batch,

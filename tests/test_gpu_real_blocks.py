@@ -73,3 +73,18 @@ def test_nan_query_reaches_only_its_block(s, at):
     imp, imp2 = _both(q, k, v)
     assert torch.equal(imp.isnan(), imp2.isnan())
     assert imp[0, :at + 1].isnan().all() and imp[0, (at | 31) + 1:].isfinite().all()
+
+
+@pytest.mark.parametrize("hq,s,d,window", [(1, 40000, 64, None), (2, 33001, 64, 700), (1, 262209, 64, 300)])
+def test_long_rows_share_blocks_and_take_turns(hq, s, d, window):
+    """Few heads and many keys: a block's stages are shared by several workgroups (scores
+    alone), sums of later launches are added, and past 262144 keys a causal output and its
+    sums take passes of their own (with a window they do not)."""
+    print(f"[gpu] long rows {hq} x {s} x {d} window={window}", flush=True)
+    q, k, v = _inputs(1, hq, 1, s, d, torch.float16)
+    imp, imp2 = _both(q, k, v, sliding_window=window)
+    assert torch.equal(imp, imp2)
+    # every row of P sums to 1: fp16 probabilities, each off by at most 2^-11 of itself or
+    # half a subnormal step, 2^-25
+    total, most = float(imp.double().sum()), window or s
+    assert abs(total - s) <= s * (2.0 ** -11 + min(most, s) * 2.0 ** -25)

@@ -79,3 +79,13 @@ def test_real_scorer_refuses_softcapping_for_fp32_models():
     with pytest.raises(NotImplementedError, match="soft-capping"):
         real_importance(model, torch.randint(0, 128, (1, 20)))
     assert model.config._attn_implementation == "eager"
+
+
+def test_attention_workspace_holds_a_round_of_workgroups():
+    """A launch that forms output and scores needs two workgroups per CU (512), whose column
+    sums take a row of keys each; one 128-query block of 8 heads is 8 of them."""
+    from nexusquant_amd import _lib
+    lib = _lib.load()
+    for hq, hkv, s in ((8, 8, 131072), (32, 8, 131072), (2, 1, 200000)):
+        rest = -(-hq * s * 12 // 256) * 256 + hkv * 64 * s * 2
+        assert lib.nq_attention_real_workspace(1, hq, hkv, s, 64) - rest >= min(512 * s * 4, hq * (s // 128) * s * 4)
