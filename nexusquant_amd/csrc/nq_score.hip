@@ -743,9 +743,11 @@ __device__ __forceinline__ void out_pv(const uint4 (&pa)[2], const char* vbuf, i
 // lane holds a query's keys, so the tile is first transposed on the matrix cores:
 // P times the slot-order permutation (sel: 1 where K slot and key meet), which is
 // exact, gives lane (c, g) key c at the queries acc_row(., g).
-// MASKED: entries outside the mask are left out again, so that a NaN row (NaN * 0)
-// reaches only keys that its query sees; query row r of the tile sees its keys
-// lo + r < key <= hi + r.
+// MASKED: entries outside the mask are left out again, because the transposition
+// spreads a NaN row (NaN * 0) over the tile; query row r of the tile sees its keys
+// lo + r < key <= hi + r.  tile_sums still adds NaN * 0 of the key 16 further on (or
+// back) in the tile: a NaN query reaches the keys it sees and the other one of each
+// such pair, key ^ 16.
 template <int DT, bool MASKED, bool WIN>
 __device__ __forceinline__ f32x4 tile_colsum(const uint4 (&pa)[2], const uint4 (&sel)[2], const uint4& ones_sel,
                                              int lo, int hi, int c, int g) {

@@ -75,6 +75,22 @@ def test_nan_query_reaches_only_its_block(s, at):
     assert imp[0, :at + 1].isnan().all() and imp[0, (at | 31) + 1:].isfinite().all()
 
 
+@pytest.mark.parametrize("s,at,window", [(300, 70, None), (300, 299, None), (2500, 130, None), (300, 37, None),
+                                         (300, 38, 20), (700, 390, 33), (700, 389, 100), (2500, 1999, 1000), (300, 5, 1)])
+@pytest.mark.parametrize("d", [64, 128])
+def test_nan_query_reaches_the_keys_it_sees_and_their_partners(s, at, window, d):
+    """Exactly the keys that the query sees, and key ^ 16 of each: the two share a row of
+    the MFMA that sums the columns."""
+    q, k, v = _inputs(1, 2, 2, s, d, torch.float16)
+    q[0, 1, at] = float("nan")
+    imp, imp2 = _both(q, k, v, sliding_window=window)
+    want = torch.zeros(s + 32, dtype=torch.bool, device=DEV)
+    seen = torch.arange(max(0, at - (window or s) + 1), at + 1, device=DEV)
+    want[seen] = True
+    want[seen ^ 16] = True
+    assert torch.equal(imp[0].isnan(), want[:s]) and torch.equal(imp2[0].isnan(), want[:s])
+
+
 @pytest.mark.parametrize("hq,s,d,window", [(1, 40000, 64, None), (2, 33001, 64, 700), (1, 262209, 64, 300)])
 def test_long_rows_share_blocks_and_take_turns(hq, s, d, window):
     """Few heads and many keys: a block's stages are shared by several workgroups (scores
