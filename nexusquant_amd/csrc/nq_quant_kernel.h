@@ -345,22 +345,31 @@ struct RowOut {
 // store instruction writes 16 runs of 64 bytes, half a cache line each; through
 // the wave's LDS buffer (swizzled as in store_rows16) it writes whole rows, 16
 // bytes a lane: instruction i stores 16-byte unit k of the wave's row rr, with
-// (rr, k) = divmod(64 i + lane, 16-byte units of a row).  row[i] is that row's token in
+// (rr, k) = divmod(64 i + lane, 16-byte units of a row or piece).  row[i] is that row's token in
 // the output and act bit i whether this launch writes it.
 // Measured (bit-identical outputs; a call's time): 16 layers x K, V fp16 [4, 8, 8192,
 // 128] evicted at 25 %: 847 -> 811 us; 4 layers bf16 [1, 8, 131072, 128] with codes
 // 1006 -> 979; 4 layers of 65521 tokens truncated at 25 %: 759 -> 726.  The rest is
 // VALU issue: about 1080 instructions per 16 rows.
+// Rows of head_dim 256 leave in four pieces of a cache line each: whole rows cost 32 KB
+// of LDS a block and 22 registers, half the waves (4 -> 2 per SIMD for values, 2 -> 1
+// for gathered keys), and are slower for it.  2 tensors of [1, 8, 32768, 256] bf16, us,
+// quad stores / whole rows / pieces: values 122 / 130 / 103, with codes 136 / 154 / 123,
+// gathered keys 203 / 252 / 151, listed keys 147 / 141 / 140.
 template <int DR>
 struct WideRows {
-    static constexpr int UR = DR / 8;   // 16-byte units per row
-    static constexpr int N = DR / 32;   // store instructions (and chunks)
+    static constexpr int P = DR > 128 ? DR / 64 : 1;  // pieces of a row, stored one after the other
+    static constexpr int UR = DR / 8;                 // 16-byte units per row
+    static constexpr int UP = UR / P;                 // and per piece
+    static constexpr int N = DR / 32 / P;             // store instructions (and chunks) per piece
     uint4* lds;
     uint32_t row[N];
     uint32_t act;
     bool all;  // every unit of the wave's rows is written
 
-    static __device__ __forceinline__ int slot(int r, int k) { return r * UR + (UR % 16 == 0 ? k ^ (4 * (r & 3)) : k); }
+    static __device__ __forceinline__ int slot(int r, int k) {
+        return r * UP + (UP % 16 == 0 ? k ^ (4 * (r & 3)) : P > 1 ? k ^ (4 * ((r >> 1) & 1)) : k);
+    }
 
     __device__ __forceinline__ void init(uint4* wave_lds, uint32_t t_out, bool active) {
         const int lane = threadIdx.x & 63;
@@ -368,19 +377,19 @@ struct WideRows {
         act = 0;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            const int src = 4 * ((64 * i + lane) / UR);  // the quad that owns the row
+            const int src = 4 * ((64 * i + lane) / UP);  // the quad that owns the row
             row[i] = (uint32_t)__shfl((int)t_out, src, 64);
             act |= (uint32_t)__shfl(active ? 1 : 0, src, 64) << i;
         }
         all = __ballot(active) == ~0ull;
     }
 
-    __device__ __forceinline__ void store(uint16_t* recon, uint32_t row0, const u32x4 (&v)[N], bool stream) const {
+    __device__ __forceinline__ void store(uint16_t* recon, uint32_t row0, int piece, const u32x4 (&v)[N], bool stream) const {
         const int lane = threadIdx.x & 63;
         u32x4* d[N];
 #pragma unroll
         for (int i = 0; i < N; ++i)
-            d[i] = reinterpret_cast<u32x4*>(recon) + (size_t)(row0 + row[i]) * UR + (64 * i + lane) % UR;
+            d[i] = reinterpret_cast<u32x4*>(recon) + (size_t)(row0 + row[i]) * UR + piece * UP + (64 * i + lane) % UP;
         if (all && stream) {
             asm volatile("" ::: "memory");  // keeps the branches' stores apart: merged, they lose the hint
 #pragma unroll
@@ -612,37 +621,37 @@ __device__ __forceinline__ void quant_row_body(const QuantArgs& a, const WideRow
     for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int i = 0; i < 8; ++i) asm("" : "+v"(x[c][i]));
-    uint4 w[DR / 32];
-#pragma unroll
-    for (int c = 0; c < DR / 32; ++c) {  // padding coordinates are not part of the output
+    auto chunk = [&](int c) {
         half2v hv[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) hv[k] = half2v{(__fp16)x[c][2 * k], (__fp16)x[c][2 * k + 1]};
-        w[c].x = __builtin_bit_cast(uint32_t, hv[0]);
-        w[c].y = __builtin_bit_cast(uint32_t, hv[1]);
-        w[c].z = __builtin_bit_cast(uint32_t, hv[2]);
-        w[c].w = __builtin_bit_cast(uint32_t, hv[3]);
-    }
+        return make_uint4(__builtin_bit_cast(uint32_t, hv[0]), __builtin_bit_cast(uint32_t, hv[1]),
+                          __builtin_bit_cast(uint32_t, hv[2]), __builtin_bit_cast(uint32_t, hv[3]));
+    };
     if constexpr (WIDE) {
         // the wave's own buffer: its LDS accesses execute in order, the barriers
         // only keep the compiler from reordering them
+        using W = WideRows<DR>;
         const int lane = threadIdx.x & 63;
 #pragma unroll
-        for (int c = 0; c < DR / 32; ++c) wide.lds[wide.slot(lane >> 2, 4 * c + q)] = w[c];
-        __builtin_amdgcn_wave_barrier();
-        u32x4 v[DR / 32];
+        for (int p = 0; p < W::P; ++p) {
 #pragma unroll
-        for (int i = 0; i < DR / 32; ++i) {
-            const int u = 64 * i + lane;
-            v[i] = *reinterpret_cast<const u32x4*>(&wide.lds[wide.slot(u / wide.UR, u % wide.UR)]);
+            for (int c = 0; c < W::N; ++c) wide.lds[wide.slot(lane >> 2, 4 * c + q)] = chunk(W::N * p + c);
+            __builtin_amdgcn_wave_barrier();
+            u32x4 v[W::N];
+#pragma unroll
+            for (int i = 0; i < W::N; ++i) {
+                const int u = 64 * i + lane;
+                v[i] = *reinterpret_cast<const u32x4*>(&wide.lds[wide.slot(u / W::UP, u % W::UP)]);
+            }
+            __builtin_amdgcn_wave_barrier();
+            wide.store(o.recon, bh * a.seq_out, p, v, a.stream_out != 0);
         }
-        __builtin_amdgcn_wave_barrier();
-        wide.store(o.recon, bh * a.seq_out, v, a.stream_out != 0);
     } else {
         if (!active) return;
         uint16_t* dst = o.recon + out_row * DR;
 #pragma unroll
-        for (int c = 0; c < DR / 32; ++c) *reinterpret_cast<uint4*>(dst + 32 * c + 8 * q) = w[c];
+        for (int c = 0; c < DR / 32; ++c) *reinterpret_cast<uint4*>(dst + 32 * c + 8 * q) = chunk(c);
     }
     }  // !PAGE
 }
@@ -658,8 +667,9 @@ __device__ __forceinline__ void store_evicted_row(const RowOut& o, const WideRow
                                                   int q, bool active, bool stream) {
     constexpr int C = D / 32;
     if (o.recon) {
-        u32x4 zero[DR / 32] = {};
-        wide.store(o.recon, row0, zero, stream);
+        const u32x4 zero[WideRows<DR>::N] = {};
+#pragma unroll
+        for (int p = 0; p < WideRows<DR>::P; ++p) wide.store(o.recon, row0, p, zero, stream);
     }
     if (!active) return;
     const size_t out_row = row0 + t_out;
@@ -758,9 +768,11 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
     uint32_t t_out = in_range ? t_raw : a.seq_out - 1u;  // idle quads recompute a valid row
     uint32_t t_in = t_out;
     bool keep = true;
-    // Whole-line stores of the reconstructions; keys with the padded RoPE layout
-    // keep the quad stores (their RoPE rows already take 24 KB of LDS a block).
-    constexpr bool WIDE = !PAGE && !(IS_KEY && DR != D);
+    // Whole-line stores of the reconstructions.  Keys with the padded RoPE layout
+    // keep the quad stores (their RoPE rows already take 24 KB of LDS a block), and so
+    // do 16-bit keys of head_dim 256 without a row selection, two waves per SIMD that
+    // the detour through LDS only delays (bf16 as above, 161 us against 173).
+    constexpr bool WIDE = !PAGE && !(IS_KEY && DR != D) && !(IS_KEY && DR == 256 && SEL == kSelNone && DT != NQ_F32);
     WideRows<DR> wide;
     if constexpr (LIST) {
         // Row list: entry t_raw of the batch row's list; the first n_kept are kept.
@@ -799,9 +811,9 @@ quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
     const bool active = in_range && (a.keep_mode == NQ_KEEP_ZERO || keep == (a.keep_mode == NQ_KEEP_WRITE_KEPT));
     if (a.keep_mode != NQ_KEEP_ZERO) keep = true;  // selected rows are quantized as they are
 
-    __shared__ uint4 out_stage[WIDE ? 4 * 16 * (DR / 8) : 1];
-    if constexpr (WIDE)
-        wide.init(out_stage + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * (16 * (DR / 8)), t_out, active);
+    constexpr int kRowUnits = 16 * WideRows<DR>::UP;  // of a wave's rows, or pieces of them
+    __shared__ uint4 out_stage[WIDE ? 4 * kRowUnits : 1];
+    if constexpr (WIDE) wide.init(out_stage + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kRowUnits, t_out, active);
 
     // Keys: the RoPE rows of the source position, loaded once for the work item
     // (pages rotate at per-page positions, loaded per sub-item).

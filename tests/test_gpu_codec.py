@@ -165,3 +165,27 @@ def test_dequantize_many_streams(D, L, key, n_t, shape):
     out = dequantize(cd, rope_base=10000.0)
     torch.cuda.synchronize()
     assert all(_same_fp16(o, r) for o, r in zip(out, rec))
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("key,mode", [(False, "plain"), (False, "list"), (False, "gather"), (True, "plain"),
+                                      (True, "list"), (True, "gather")])
+@pytest.mark.parametrize("s", [1, 63, 1000, 11003])
+def test_head_dim_256_rows_stored_in_pieces(dt, key, mode, s):
+    """The quantizer's reconstruction, stored a cache line at a time (nontemporally at 11003
+    rows), is what its codes decode to."""
+    from nexusquant_amd.codec import dequantize
+    from nexusquant_amd.ops import quantize_tensors
+    print(f"[gpu] pieces {dt} key={key} {mode} s={s}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(s)
+    xs = [torch.randn(1, 3, s, 256, generator=g, device=DEV).to(dt) for _ in range(2)]
+    kw = {}
+    keep = torch.rand(1, s, generator=g, device=DEV) < 0.6
+    kept, evicted = keep[0].nonzero()[:, 0], (~keep[0]).nonzero()[:, 0].flip(0)
+    if mode == "list":
+        kw = dict(keep=keep.to(torch.uint8), order=torch.cat([kept, evicted]).int().unsqueeze(0), n_kept=keep.sum(1).int())
+    elif mode == "gather":
+        kw = dict(gather=torch.cat([kept, torch.tensor([s - 1], device=DEV)]).int().unsqueeze(0))
+    for levels in (8, 16):
+        rec, codes = quantize_tensors(xs, is_key=key, levels=levels, codes=True, **kw)
+        assert all(_same_fp16(o, r) for o, r in zip(dequantize(codes, rope_base=10000.0), rec))

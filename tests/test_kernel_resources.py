@@ -1,5 +1,6 @@
 """Resources of the built kernels, from the metadata that the compiler writes beside them."""
 
+import re
 import struct
 
 import pytest
@@ -60,3 +61,19 @@ def test_attention_kernels_keep_their_waves(kernels):
     for name, k in kernels.items():
         if "paged_attn_kernel" in name:
             assert k[".vgpr_count"] <= (256 if "ILi256E" in name else 128), name
+
+
+def test_quantizer_kernels_leave_room_for_their_waves(kernels):
+    """LDS of a block and registers: three blocks of a CU's 160 KB everywhere, four at head_dim 256,
+    and there 2 waves per SIMD for keys and 3 for values (gathered keys of 16 levels never had 2)."""
+    seen = 0
+    for name, k in kernels.items():
+        m = re.search(r"quant_rows_kernelILi(\d+)ELi(\d+)ELb([01])ELi(\d)ELi(\d+)ELb([01])ELi(\d)E", name)
+        if not m:
+            continue
+        seen += 1
+        head_dim, levels, is_key, sel = int(m[5]), int(m[2]), m[3] == "1", int(m[7])
+        assert k[".group_segment_fixed_size"] <= (40960 if head_dim == 256 else 49152), name
+        if head_dim == 256 and not (is_key and levels == 16 and sel == 2):
+            assert k[".vgpr_count"] + k[".agpr_count"] <= (256 if is_key else 168), name
+    assert seen > 100
