@@ -175,7 +175,9 @@ int nq_score_keykey_noalloc(const void* keys, int32_t dtype, int32_t batch, int3
  * is monotone non-decreasing -- Gemma-2's soft-capping
  * round(round(tanh(round(x / cap))) * cap), built by the host with the
  * framework's own ops.  workspace: at least
- * nq_score_real_workspace(batch, q_heads, seq) bytes (caller owned).
+ * nq_score_real_workspace(batch, q_heads, seq) bytes (caller owned): 12 bytes
+ * per query row, and nq_real_block_sums_bytes(batch, q_heads, seq, 0) for the
+ * column sums of 128-query blocks, which fp32 inputs do not need.
  *
  * Replaces: NexusQuantEvict._score_importance_real   pipeline.py:784-836
  *           (eager_attention_forward + repeat_kv, transformers 5.15.0
@@ -184,6 +186,15 @@ int nq_score_keykey_noalloc(const void* keys, int32_t dtype, int32_t batch, int3
  *            mask masking_utils.py:92-101)
  */
 int64_t nq_score_real_workspace(int32_t batch, int32_t q_heads, int32_t seq);
+/*
+ * The part of nq_score_real_workspace (with_output 0) or of
+ * nq_attention_real_workspace (1) that holds column sums of 128-query blocks: all
+ * blocks' up to 128 MiB, else as many as fit that, with_output as many as make
+ * 512 workgroups if they fit 512 MiB; one block's at least.  A call that forms no
+ * column sums of blocks (fp32 scores, attention without importance) takes a
+ * workspace without it.
+ */
+int64_t nq_real_block_sums_bytes(int32_t batch, int32_t q_heads, int32_t seq, int32_t with_output);
 int nq_score_real(const void* q, const void* k, int32_t dtype, int32_t batch, int32_t q_heads,
                   int32_t kv_heads, int32_t seq, int32_t head_dim, float scaling, int32_t sliding_window,
                   const uint16_t* logit_map, float* importance, void* workspace, int64_t workspace_bytes,
@@ -198,8 +209,9 @@ int nq_score_real(const void* q, const void* k, int32_t dtype, int32_t batch, in
  * in fp32 on the matrix cores.  fp16 / bf16, head_dim 64 or 128, 16-byte aligned
  * tensors; v [batch, kv_heads, seq, head_dim]; sliding_window and logit_map as
  * for nq_score_real.  workspace:
- * nq_attention_real_workspace bytes (nq_score_real's and V transposed with the
- * keys of each 32-key block in the accumulator's order).
+ * nq_attention_real_workspace bytes (12 per query row, V transposed with the keys
+ * of each 32-key block in the accumulator's order, and, with importance,
+ * nq_real_block_sums_bytes(batch, q_heads, seq, 1)).
  *
  * Replaces: eager_attention_forward (transformers modeling_llama.py:179-213) in
  *           the scoring forward of _score_importance_real  pipeline.py:784-836

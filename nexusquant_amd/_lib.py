@@ -107,6 +107,7 @@ SIGNATURES = {
     "nq_codes_to_int8": ([ctypes.POINTER(CodesDesc), _I32, _P], ctypes.c_int),
     "nq_delta_encode": ([_P, _P, _I32, _I32, _I32, _I32, _P], ctypes.c_int),
     "nq_delta_decode": ([_P, _P, _I32, _I32, _I32, _I32, _P], ctypes.c_int),
+    "nq_real_block_sums_bytes": ([_I32, _I32, _I32, _I32], _I64),
     "nq_score_real_workspace": ([_I32, _I32, _I32], _I64),
     "nq_score_real": ([_P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _F32, _I32, _P, _P, _P, _I64, _P],
                       ctypes.c_int),

@@ -1215,9 +1215,14 @@ static hipError_t dispatch_real_d(int d, const RealArgs& a, float* partial, hipS
 
 }  // namespace nq
 
+extern "C" int64_t nq_real_block_sums_bytes(int32_t batch, int32_t q_heads, int32_t seq, int32_t with_output) {
+    if (batch <= 0 || q_heads <= 0 || seq <= 0) return 0;
+    return nq::partial_bytes((int64_t)batch * q_heads, seq, with_output != 0);
+}
+
 extern "C" int64_t nq_score_real_workspace(int32_t batch, int32_t q_heads, int32_t seq) {
     if (batch <= 0 || q_heads <= 0 || seq <= 0) return 0;
-    return nq::stats_bytes(batch, q_heads, seq) + nq::partial_bytes((int64_t)batch * q_heads, seq, false);
+    return nq::stats_bytes(batch, q_heads, seq) + nq_real_block_sums_bytes(batch, q_heads, seq, 0);
 }
 
 extern "C" int nq_score_real(const void* q, const void* k, int32_t dtype, int32_t batch, int32_t q_heads,
@@ -1236,7 +1241,8 @@ extern "C" int nq_score_real(const void* q, const void* k, int32_t dtype, int32_
                  "nq_score_real: head_dim %d unsupported (64, 96, 128, 256)", head_dim);
     NQ_CHECK_ARG(dtype == NQ_F16 || dtype == NQ_BF16 || dtype == NQ_F32, "nq_score_real: bad dtype");
     if (seq == 0) return NQ_OK;
-    const int64_t need = nq_score_real_workspace(batch, q_heads, seq);
+    const int64_t need = nq_score_real_workspace(batch, q_heads, seq) -
+                         (dtype == NQ_F32 ? nq_real_block_sums_bytes(batch, q_heads, seq, 0) : 0);
     NQ_CHECK_ARG(workspace_bytes >= need, "nq_score_real: workspace %lld bytes < %lld",
                  (long long)workspace_bytes, (long long)need);
     RealArgs a;
@@ -1271,7 +1277,7 @@ extern "C" int64_t nq_attention_real_workspace(int32_t batch, int32_t q_heads, i
     if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || seq <= 0 || head_dim <= 0) return 0;
     const int64_t stats = nq::stats_bytes(batch, q_heads, seq);
     const int64_t vt = (int64_t)batch * kv_heads * head_dim * nq::padded_keys(seq) * 2;
-    return stats + vt + nq::partial_bytes((int64_t)batch * q_heads, seq, true);
+    return stats + vt + nq_real_block_sums_bytes(batch, q_heads, seq, 1);
 }
 
 extern "C" int nq_attention_real(const void* q, const void* k, const void* v, int32_t dtype, int32_t batch,
@@ -1291,7 +1297,8 @@ extern "C" int nq_attention_real(const void* q, const void* k, const void* v, in
                  "nq_attention_real: tensors must be 16-byte aligned");
     if (seq == 0) return NQ_OK;
     NQ_CHECK_ARG((int64_t)seq * head_dim < (1ll << 31), "nq_attention_real: seq too long");
-    const int64_t need = nq_attention_real_workspace(batch, q_heads, kv_heads, seq, head_dim);
+    const int64_t need = nq_attention_real_workspace(batch, q_heads, kv_heads, seq, head_dim) -
+                         (importance ? 0 : nq_real_block_sums_bytes(batch, q_heads, seq, 1));
     NQ_CHECK_ARG(workspace_bytes >= need, "nq_attention_real: workspace %lld bytes < %lld",
                  (long long)workspace_bytes, (long long)need);
     RealArgs a;

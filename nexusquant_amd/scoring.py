@@ -100,6 +100,8 @@ def score_real_accumulate(query: torch.Tensor, key: torch.Tensor, importance: to
     k = key.contiguous()
     dev = q.device
     ws_bytes = lib.nq_score_real_workspace(b, hq, s)
+    if q.dtype == torch.float32:  # its kernels sum no blocks
+        ws_bytes -= lib.nq_real_block_sums_bytes(b, hq, s, 0)
     ws = workspace(dev, ws_bytes)
     lm = None if softcap is None else logit_map(q.dtype, softcap, dev)
     with torch.cuda.device(dev):
@@ -131,6 +133,8 @@ def attention_real(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, 
     dev = q.device
     out = torch.empty_like(q)
     ws_bytes = lib.nq_attention_real_workspace(b, hq, hkv, s, d)
+    if importance is None:
+        ws_bytes -= lib.nq_real_block_sums_bytes(b, hq, s, 1)
     ws = workspace(dev, ws_bytes)
     lm = None if softcap is None else logit_map(q.dtype, softcap, dev)
     with torch.cuda.device(dev):

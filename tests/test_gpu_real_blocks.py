@@ -104,3 +104,18 @@ def test_long_rows_share_blocks_and_take_turns(hq, s, d, window):
     # half a subnormal step, 2^-25
     total, most = float(imp.double().sum()), window or s
     assert abs(total - s) <= s * (2.0 ** -11 + min(most, s) * 2.0 ** -25)
+
+
+def test_calls_without_block_sums_hold_no_memory_for_them():
+    """fp32 scores and attention without importance: 12 bytes per query row (and V transposed)."""
+    from nexusquant_amd import ops
+    from nexusquant_amd.scoring import attention_real, score_real_accumulate
+    q, k, v = _inputs(1, 4, 2, 3000, 64, torch.float16)
+    for call, most in ((lambda: score_real_accumulate(q.float(), k.float(), torch.zeros(1, 3000, device=DEV), 0.125),
+                        12 * 4 * 3000 + 256),
+                       (lambda: attention_real(q, k, v, 0.125), 12 * 4 * 3000 + 256 + 2 * 64 * 3008 * 2)):
+        ops.release_workspaces()
+        call()
+        # the cached workspace is rounded up to 1 MiB; the blocks' sums would take 1.1 more
+        assert sum(t.numel() for t in ops._workspaces.values()) == -(-most // (1 << 20)) << 20
+    ops.release_workspaces()
