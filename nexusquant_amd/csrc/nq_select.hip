@@ -44,7 +44,7 @@ __device__ __forceinline__ uint32_t order_key(float f) {
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-// Inclusive block scan of one value per thread.  Uses lds[0 .. 31] and ends
+// Inclusive block scan of one value per thread.  Uses lds[0 .. kSelWaves - 1] and ends
 // without a barrier: the caller puts one before lds is written again.
 __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* lds) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;

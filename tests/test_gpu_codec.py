@@ -189,3 +189,21 @@ def test_head_dim_256_rows_stored_in_pieces(dt, key, mode, s):
     for levels in (8, 16):
         rec, codes = quantize_tensors(xs, is_key=key, levels=levels, codes=True, **kw)
         assert all(_same_fp16(o, r) for o, r in zip(dequantize(codes, rope_base=10000.0), rec))
+
+
+@pytest.mark.parametrize("D,L,key,n_t,shape", [(128, 8, True, 33, (1, 8, 637)), (128, 4, False, 17, (1, 8, 1001)),
+                                               (96, 8, True, 11, (1, 16, 1025)), (64, 2, True, 33, (1, 8, 1283)),
+                                               (256, 16, False, 9, (1, 8, 1000))])
+def test_dequantize_large_launches_end_in_a_cut_tile(D, L, key, n_t, shape):
+    """32 MB and more, stored nontemporally, with rows left over past the last whole tile: the
+    same bytes as one launch per tensor, which stays below that size."""
+    from nexusquant_amd.codec import dequantize
+    from nexusquant_amd.ops import quantize_tensors
+    print(f"[gpu] dequant cut tile D={D} L={L} key={key} n={n_t} {shape}", flush=True)
+    one = 2 * shape[0] * shape[1] * shape[2] * D
+    assert one < 32 << 20 <= n_t * one and shape[2] % 64
+    g = torch.Generator(device=DEV).manual_seed(D + L)
+    xs = [torch.randn(*shape, D, generator=g, device=DEV).half() for _ in range(n_t)]
+    _, cd = quantize_tensors(xs, is_key=key, levels=L, recon=False, codes=True)
+    for c, got in zip(cd, dequantize(cd)):
+        assert torch.equal(got, dequantize([c])[0])
