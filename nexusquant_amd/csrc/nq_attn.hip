@@ -30,11 +30,12 @@
 //     and divides by the softmax sum.
 //
 // What bounds it: the latency of a unit's loads and of the three phases one after
-// another; the vector ALUs are busy about half the time (3550 instructions a wave;
-// 4600 when the keys were decoded on them, a quad of lanes a token), the page bytes
-// move at 2.9 TB/s.  Measured against that form, call between events, us: 64/8 heads
-// x 131072 tokens 121.3 -> 116.5; 32/32 heads x 4 x 8192 100.7 -> 99.5; 32/8 bf16, 8
-// ragged rows up to 4096 40.0 -> 34.0, and 26.8 with the shorter chunks below.
+// another.  Counters at 64/8 heads x 131072 tokens: the vector ALUs are busy 57 % of the
+// time (3670 instructions a wave), the matrix cores 8 %, waves wait on memory for 32 % of
+// theirs; the page bytes move at 2.9 TB/s.  A call between events, us, against the form
+// that decoded the keys on the vector ALUs, a quad of lanes a token: that size 98.5 ->
+// 92.4; 32/32 heads x 4 x 8192 71.7 -> 67.2; 32/8 heads bf16 x 32768 35.1 -> 30.7, and 8
+// ragged rows up to 4096 33.5 -> 20.7 with the shorter chunks below.
 //
 // Chunks are 512 tokens when that makes enough workgroups, else shorter: the caller
 // halves them down to 64 tokens while chunks x kv heads is below two per CU (512).

@@ -350,7 +350,8 @@ struct RowOut {
 // Measured (bit-identical outputs; a call's time): 16 layers x K, V fp16 [4, 8, 8192,
 // 128] evicted at 25 %: 847 -> 811 us; 4 layers bf16 [1, 8, 131072, 128] with codes
 // 1006 -> 979; 4 layers of 65521 tokens truncated at 25 %: 759 -> 726.  The rest is
-// VALU issue: about 1080 instructions per 16 rows.
+// VALU issue: 1097 instructions per 16 rows of keys and 1043 of values (counters of the
+// 80-layer launches at 131072 tokens; 1082 and 1025 with quad stores).
 // Rows of head_dim 256 leave in four pieces of a cache line each: whole rows cost 32 KB
 // of LDS a block and 22 registers, half the waves (4 -> 2 per SIMD for values, 2 -> 1
 // for gathered keys), and are slower for it.  2 tensors of [1, 8, 32768, 256] bf16, us,
