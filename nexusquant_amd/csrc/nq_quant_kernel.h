@@ -343,23 +343,24 @@ struct RowOut {
 
 // Whole-line stores of a wave's 16 reconstructed rows.  In the quad layout a
 // store instruction writes 16 runs of 64 bytes, half a cache line each; through
-// the wave's LDS buffer (swizzled as in store_rows16) it writes whole rows, 16
-// bytes a lane: instruction i stores 16-byte unit k of the wave's row rr, with
-// (rr, k) = divmod(64 i + lane, 16-byte units of a row or piece).  row[i] is that row's token in
+// the wave's LDS buffer (swizzled) it writes whole lines, 16 bytes a lane.  Rows of
+// 128 and 256 coordinates pass in pieces of 64, one 128-byte line each, shorter ones
+// whole: instruction i stores 16-byte unit k of the wave's row rr, with
+// (rr, k) = divmod(64 i + lane, 16-byte units of a piece).  row[i] is that row's token in
 // the output and act bit i whether this launch writes it.
 // Measured (bit-identical outputs; a call's time): 16 layers x K, V fp16 [4, 8, 8192,
 // 128] evicted at 25 %: 847 -> 811 us; 4 layers bf16 [1, 8, 131072, 128] with codes
-// 1006 -> 979; 4 layers of 65521 tokens truncated at 25 %: 759 -> 726.  The rest is
-// VALU issue: 1097 instructions per 16 rows of keys and 1043 of values (counters of the
-// 80-layer launches at 131072 tokens; 1082 and 1025 with quad stores).
-// Rows of head_dim 256 leave in four pieces of a cache line each: whole rows cost 32 KB
-// of LDS a block and 22 registers, half the waves (4 -> 2 per SIMD for values, 2 -> 1
-// for gathered keys), and are slower for it.  2 tensors of [1, 8, 32768, 256] bf16, us,
-// quad stores / whole rows / pieces: values 122 / 130 / 103, with codes 136 / 154 / 123,
-// gathered keys 203 / 252 / 151, listed keys 147 / 141 / 140.
+// 1006 -> 979; 4 layers of 65521 tokens truncated at 25 %: 759 -> 726, these with whole
+// rows.  The rest is VALU issue.
+// Pieces, not whole rows, because whole rows cost 16 (128) or 32 KB (256) of LDS a block
+// and 8 or 22 registers; at 256 that halves the waves (4 -> 2 per SIMD for values, 2 ->
+// 1 for gathered keys).  us, quad stores / whole rows / pieces: 2 tensors of [1, 8, 32768,
+// 256] bf16, values 122 / 130 / 103, with codes 136 / 154 / 123, gathered keys 203 / 252 /
+// 151, listed keys 147 / 141 / 140; kernel, 32 tensors of 6153 gathered rows x 8 x 128
+// fp16, values 162 / 172 / 163; 2 of [1, 8, 32768, 128] fp32, values 86 / 67 / 60.
 template <int DR>
 struct WideRows {
-    static constexpr int P = DR > 128 ? DR / 64 : 1;  // pieces of a row, stored one after the other
+    static constexpr int P = DR >= 128 ? DR / 64 : 1;  // pieces of a row, stored one after the other
     static constexpr int UR = DR / 8;                 // 16-byte units per row
     static constexpr int UP = UR / P;                 // and per piece
     static constexpr int N = DR / 32 / P;             // store instructions (and chunks) per piece
@@ -714,8 +715,10 @@ constexpr int kSelGather = 2;
 // Keys with the padded RoPE layout (head_dim 96): the row-list instantiation
 // (mask eviction, the Phi-3 workload) fits 4 waves per SIMD without spills
 // (126 VGPRs); the others keep their natural 3 waves rather than spill at 4.
+// Values of head_dim 256 up to 8 levels fit 4 as well (114 to 125; left alone the
+// compiler takes up to 137 for 2 and 4 levels, 3 waves).
 template <int D, int L, bool IS_KEY, int DT, int DR, bool PAGE = false, int SEL = kSelNone>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((IS_KEY && !PAGE && DR != D && SEL == kSelList) ? 4 : 1))) void
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(((IS_KEY && !PAGE && DR != D && SEL == kSelList) || (!IS_KEY && !PAGE && DR == 256 && L <= 8)) ? 4 : 1))) void
 quant_rows_kernel(QuantArgs a, const uint64_t* __restrict__ tab_src,
                                                          const uint64_t* __restrict__ tab_recon,
                                                          const uint64_t* __restrict__ tab_syms,

@@ -64,8 +64,8 @@ def test_attention_kernels_keep_their_waves(kernels):
 
 
 def test_quantizer_kernels_leave_room_for_their_waves(kernels):
-    """LDS of a block and registers: three blocks of a CU's 160 KB everywhere, four at head_dim 256,
-    and there 2 waves per SIMD for keys and 3 for values (gathered keys of 16 levels never had 2)."""
+    """LDS of a block: four to a CU's 160 KB, three of padded keys.  Registers at head_dim 256: 4 waves
+    per SIMD for values up to 8 levels and 3 past that, 2 for keys (gathered keys of 16 levels have 1)."""
     seen = 0
     for name, k in kernels.items():
         m = re.search(r"quant_rows_kernelILi(\d+)ELi(\d+)ELb([01])ELi(\d)ELi(\d+)ELb([01])ELi(\d)E", name)
@@ -73,7 +73,8 @@ def test_quantizer_kernels_leave_room_for_their_waves(kernels):
             continue
         seen += 1
         head_dim, levels, is_key, sel = int(m[5]), int(m[2]), m[3] == "1", int(m[7])
-        assert k[".group_segment_fixed_size"] <= (40960 if head_dim == 256 else 49152), name
+        assert k[".group_segment_fixed_size"] <= (49152 if head_dim == 96 and is_key else 40960), name
         if head_dim == 256 and not (is_key and levels == 16 and sel == 2):
-            assert k[".vgpr_count"] + k[".agpr_count"] <= (256 if is_key else 168), name
+            registers = 256 if is_key else 168 if levels == 16 else 128
+            assert k[".vgpr_count"] + k[".agpr_count"] <= registers, name
     assert seen > 100
