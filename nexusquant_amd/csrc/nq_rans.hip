@@ -82,6 +82,10 @@ __global__ __launch_bounds__(kHistThreads) void rans_hist_kernel(const int8_t* c
 constexpr int kHistSmallBins = 9;
 constexpr int kHistSmallLoads = 4;  // 16-byte loads per lane in flight: 64 codes between flushes
                                     // (8 in flight, flushed every 4, measured the same)
+// Codes up to which its blocks have 256 threads: a few blocks end sooner than one of
+// 1024 (9 bins, us a call: 16384 and 131072 codes 5.4 and 5.6 -> 4.2 to 4.8; 1 M codes 7.0 with
+// 256 threads, 6.0 with 1024).
+constexpr int64_t kHistSmallCodes = 1 << 18;
 
 __global__ __launch_bounds__(kHistThreads) void rans_hist_small_kernel(const int8_t* codes, int64_t n, int L, uint32_t* hist) {
     __shared__ uint32_t h[kHistSmallBins];
@@ -108,8 +112,8 @@ __global__ __launch_bounds__(kHistThreads) void rans_hist_small_kernel(const int
     };
     const uint4* const v = reinterpret_cast<const uint4*>(codes);
     const int64_t n16 = n / 16;
-    const int64_t stride = (int64_t)gridDim.x * kHistThreads;
-    int64_t g = (int64_t)blockIdx.x * kHistThreads + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     for (; g + (kHistSmallLoads - 1) * stride < n16; g += kHistSmallLoads * stride) {
         uint4 w[kHistSmallLoads];
 #pragma unroll
@@ -766,9 +770,11 @@ extern "C" int nq_rans_histogram(const int8_t* codes, int64_t n, int32_t levels,
                  (long long)n);
     NQ_CHECK_ARG(((uintptr_t)codes & 15) == 0, "nq_rans_histogram: codes must be 16-byte aligned");
     if (n == 0) return NQ_OK;
-    const int64_t blocks = std::min<int64_t>((n + kHistThreads * 16 - 1) / (kHistThreads * 16), kHistBlocks);
-    if (2 * levels + 1 <= kHistSmallBins)
-        hipLaunchKernelGGL(rans_hist_small_kernel, dim3((uint32_t)blocks), dim3(kHistThreads), 0, (hipStream_t)stream, codes, n,
+    const bool small = 2 * levels + 1 <= kHistSmallBins;
+    const int threads = small && n <= kHistSmallCodes ? 256 : kHistThreads;
+    const int64_t blocks = std::min<int64_t>((n + threads * 16 - 1) / (threads * 16), kHistBlocks);
+    if (small)
+        hipLaunchKernelGGL(rans_hist_small_kernel, dim3((uint32_t)blocks), dim3(threads), 0, (hipStream_t)stream, codes, n,
                            levels, hist);
     else
         hipLaunchKernelGGL(rans_hist_kernel, dim3((uint32_t)blocks), dim3(kHistThreads), 0, (hipStream_t)stream, codes, n,

@@ -208,3 +208,14 @@ def test_histogram_at_the_grid_edges(levels, n):
     c = (torch.randn(n, device="cuda:0", generator=g) * levels / 3).round().clamp(-levels, levels).to(torch.int8)
     want = torch.bincount((c.to(torch.int32) + levels), minlength=2 * levels + 1).cpu().numpy()
     assert np.array_equal(_code_counts(c, levels), want)
+
+
+@pytest.mark.parametrize("levels", [2, 4])
+@pytest.mark.parametrize("n", [255, 4095, 4096, 4097, (1 << 18) - 1, 1 << 18, (1 << 18) + 1])
+def test_small_histograms_block_sizes(levels, n):
+    """Blocks of 256 threads up to 2^18 codes, of 1024 past that."""
+    from nexusquant_amd.entropy import _code_counts
+    g = torch.Generator(device="cuda:0").manual_seed(n + levels)
+    c = torch.randint(-levels, levels + 1, (n,), device="cuda:0", generator=g, dtype=torch.int8)
+    want = torch.bincount((c.to(torch.int32) + levels), minlength=2 * levels + 1).cpu().numpy()
+    assert np.array_equal(_code_counts(c, levels), want)
